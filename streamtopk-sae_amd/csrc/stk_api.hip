@@ -183,6 +183,8 @@ struct ExactPlan {
     bool large;                  // mainl_kernel (B >= kLargeMinB) instead of main_kernel
     bool xch;                    // main_kernel exchanges thresholds after its first tile (no sample pass)
     int NB, cap, lq;             // lq: main_kernel's LDS queue keys per row
+    int S;                       // main_kernel: 128-byte sub-steps of a row per step
+    int xper;                    // main_kernel: exchanged maxima per row and workgroup
     int64_t nbc, num_tiles, tpw;
     int nwg;                     // main_kernel: W ranges; mainl_kernel: nr (grid = nbc * nr)
     bool sample;
@@ -201,6 +203,10 @@ static ExactPlan make_exact_plan(int64_t B, int64_t d, int64_t F, int64_t k, int
     p.num_tiles = cdiv(F, kTileLatents);
     p.large = B >= kLargeMinB;
     p.lq = 0;
+    p.S = 1;
+    p.xper = 1;
+    const int64_t nds = cdiv(d, dtype == STK_DTYPE_F32 ? 32 : 64);   // 128-byte sub-steps of d, the last maybe partial
+    int64_t wg_latents = 0;      // main_kernel: latents of a workgroup (at most)
     if (p.large) {
         // 256-row blocks; W ranges a multiple of 8 so each range's row blocks share an XCD
         p.NB = kLargeRows / 32;
@@ -214,26 +220,60 @@ static ExactPlan make_exact_plan(int64_t B, int64_t d, int64_t F, int64_t k, int
         p.tpw = cdiv(p.num_tiles, nr);
         p.nwg = (int)nr;
     } else {
+        // Tiles of 256 / S latents, S sub-steps of d per step (split over the
+        // waves; TileStream): the same bytes of W per step.  The S with the
+        // fewest steps on the busiest workgroup is taken, a tile's epilogue
+        // counted as two steps; the smallest such S, as each split adds a
+        // reduction.  S * NB <= 4 (X's share of the LDS ring), so more than 64
+        // rows split into more row blocks, which then share W through L2.  At
+        // least three steps per tile: with fewer, the reduction and the
+        // pipeline's start outweigh them.  Measured (bf16, main_kernel): B = 1,
+        // d = 768, F = 16384 S = 1 20.1 us, S = 4 13.7; B = 128, d = 2048,
+        // F = 8192 S = 1 51.4, S = 2 25.4.
+        // The workgroups' ranges of latents differ by at most kRangeUnit, so
+        // that no CU idles through a last tile that others hold (B = 200,
+        // d = 1024, F = 100003: 99.6 us with whole tiles, 91.4 so).
         const int64_t bblocks = cdiv(B > 0 ? B : 1, 32);
-        p.NB = (int)(bblocks < 4 ? bblocks : 4);
-        if (p.NB == 3) p.NB = 4;
-        p.nbc = cdiv(B, 32 * p.NB);
-        int64_t nwg = ncu / (p.nbc > 0 ? p.nbc : 1);
-        if (nwg < 1) nwg = 1;
-        if (nwg > p.num_tiles) nwg = p.num_tiles;
-        p.tpw = cdiv(p.num_tiles, nwg);
-        p.nwg = (int)cdiv(p.num_tiles, p.tpw);
+        const int64_t nu = cdiv(F, kRangeUnit);
+        int64_t best = INT64_MAX;
+        for (int S = 1; S <= 4; S *= 2) {
+            if (S > 1 && nds < 3 * S) break;
+            const int64_t T = kTileLatents / S;
+            int64_t NB = bblocks < 4 / S ? bblocks : 4 / S;
+            if (NB == 3) NB = 4;
+            const int64_t nbc = cdiv(B, 32 * NB);
+            int64_t nwg = ncu / (nbc > 0 ? nbc : 1);
+            if (nwg > cdiv(F, T)) nwg = cdiv(F, T);
+            if (nwg < 1) nwg = 1;
+            const int64_t lat = cdiv(nu, nwg) * kRangeUnit, tiles = cdiv(lat, T);
+            const int64_t cost = tiles * (cdiv(nds, S) + 2);
+            if (cost < best) {
+                best = cost;
+                p.S = S;
+                p.NB = (int)NB;
+                p.nbc = nbc;
+                p.nwg = (int)nwg;
+                p.tpw = tiles;
+                wg_latents = lat;
+            }
+        }
+        // as many maxima per workgroup as fit the owners' polls (256 words): a
+        // small dictionary then exchanges thresholds for k up to F / 32.  (With
+        // fewer maxima than k and no sample pass, below 2^14 latents, every
+        // score was a candidate: B = 128, d = 2048, F = 8192, k = 64 took 391
+        // us, 33 us so.)
+        while (p.xper * 2 <= kMainWaves / p.S && p.nwg * p.xper * 2 <= 256) p.xper *= 2;
     }
 
     // The thresholds come from the streaming kernel's own first tiles (each
     // row's k-th largest of the n maxima its workgroups publish, each over m
-    // latents: n = nwg, m = 256 below 512 rows; n = kLXchPerWg * W ranges,
+    // latents: n = nwg * xper, m = 256 / (S * xper) below 512 rows; n = kLXchPerWg * W ranges,
     // m = 64 above) or from a sample pass of nsamp latents (whose k-th is the
     // threshold).  A latent passes the exchange's threshold with probability
     // about -ln(1 - k / n) / m and the sample's about k / nsamp.  The exchange
     // is taken when it passes at most as many (up to twice as many below 512
-    // rows, where it also saves the two launches of the sample and threshold
-    // passes, a larger share of the call); it needs n > k (n = k is the
+    // rows with one maximum per workgroup, where it also saves the two launches
+    // of the sample and threshold passes, a larger share of the call); it needs n > k (n = k is the
     // minimum of all maxima) and, below 512 rows, at least kXchMinWg
     // workgroups.  Measured (B = 512-2048, d = 2048-4096, k = 64-128): the
     // exchange was 3-8 % faster where it passes fewer latents, 1-4 % slower
@@ -243,18 +283,18 @@ static ExactPlan make_exact_plan(int64_t B, int64_t d, int64_t F, int64_t k, int
     {
         // mainl_kernel: the W ranges that hold tiles (main_kernel has no empty workgroup)
         const int64_t nfull = p.large ? cdiv(p.num_tiles, p.tpw) : p.nwg;
-        const int64_t n = p.large ? nfull * kLXchPerWg : p.nwg;
-        const double m = p.large ? 64.0 : 256.0;
+        const int64_t n = p.large ? nfull * kLXchPerWg : (int64_t)p.nwg * p.xper;
+        const double m = p.large ? 64.0 : (double)(kTileLatents / p.S / p.xper);
         // n = k still bounds the k-th score; without a sample pass (small F)
         // that weak bound beats none.  Only workgroups with a first tile take
         // part (mainl_kernel's W ranges past the last tile are empty when F is
         // small); they publish the maxima and own the rows.
         bool ok = (F < kSampleMinF ? n >= k : n > k) &&
-                  (p.large ? n <= 512 : (p.nwg >= kXchMinWg && p.nwg <= 256));
+                  (p.large ? n <= 512 : (p.nwg >= kXchMinWg && n <= 256));
         if (ok && F >= kSampleMinF) {
             const double px = -std::log1p(-(double)k / (double)n) / m;
             const double ps = (double)k / (double)samp_n;
-            ok = px <= (p.large ? 1.0 : 2.0) * ps;
+            ok = px <= (p.large || p.xper > 1 ? 1.0 : 2.0) * ps;
         }
         p.xch = ok && !hooks.no_xch;
     }
@@ -272,7 +312,6 @@ static ExactPlan make_exact_plan(int64_t B, int64_t d, int64_t F, int64_t k, int
     // ranges to fill the device
     p.ksplit = 1;
     p.snb = 1;
-    const int64_t nds = cdiv(d, dtype == STK_DTYPE_F32 ? 32 : 64);   // d-steps, the last maybe partial
     if (p.large && p.sample) {
         const int64_t wgs = p.nbc * (p.nsamp / kTileLatents);
         int64_t ks = cdiv(ncu, wgs);
@@ -301,14 +340,15 @@ static ExactPlan make_exact_plan(int64_t B, int64_t d, int64_t F, int64_t k, int
         // maxima over 256 latents each: a latent passes with probability
         // about -ln(1 - k / nwg) / 256, so a workgroup expects
         // -ln(1 - k / nwg) * tpw survivors per row.
-        const int lq_max = main_lds_queue(p.NB, (int)k);
+        const int lq_max = main_lds_queue(p.NB, p.S, (int)k);
         int lq = lq_max;
         p.expect_seg = p.cap;
         if (p.sample || p.xch) {
             int64_t expect;
             if (p.xch) {
-                const double q = std::fmin((double)k / (double)p.nwg, 0.9);
-                expect = (int64_t)std::ceil(-std::log1p(-q) * (double)p.tpw);
+                const double n = (double)p.nwg * p.xper, m = (double)(kTileLatents / p.S) / p.xper;
+                const double q = std::fmin((double)k / n, 0.9);
+                expect = (int64_t)std::ceil(-std::log1p(-q) / m * (double)wg_latents);
             } else {
                 expect = cdiv(k * F / p.nsamp, p.nwg);
             }
@@ -350,7 +390,7 @@ static ExactPlan make_exact_plan(int64_t B, int64_t d, int64_t F, int64_t k, int
     if (p.xch) {
         // [nbc][bt][words per row]
         const size_t bt = p.large ? (size_t)kLargeRows : 32 * (size_t)p.NB;
-        const size_t per_row = p.large ? (size_t)cdiv(p.num_tiles, p.tpw) * kLXchPerWg : (size_t)p.nwg;
+        const size_t per_row = p.large ? (size_t)cdiv(p.num_tiles, p.tpw) * kLXchPerWg : (size_t)p.nwg * p.xper;
         p.off_xmax = off;
         off = align256(off + (size_t)p.nbc * bt * per_row * 8);
         p.off_xthr = off;
@@ -512,7 +552,6 @@ static int run_exact(const ExactPlan& p, const TestHooks& hooks, const void* X, 
         std::memset(&ma, 0, sizeof ma);
         ma.X = X; ma.W = W; ma.bias = b; ma.B = B; ma.d = d; ma.F = F;
         ma.k = (int)k; ma.cap = p.cap;
-        ma.num_tiles = p.num_tiles; ma.tiles_per_wg = p.tpw;
         ma.thr0 = p.xch ? nullptr : thr;
         ma.sampled = p.sample ? 1 : 0;
         ma.samp_log2 = p.samp_log2;
@@ -525,12 +564,13 @@ static int run_exact(const ExactPlan& p, const TestHooks& hooks, const void* X, 
         ma.epoch = epoch;
         ma.cur = cur;
         ma.xch = p.xch ? 1 : 0;
+        ma.xper = p.xper;
         ma.xmax = (uint64_t*)(ws + p.off_xmax);
         ma.xthr = (uint64_t*)(ws + p.off_xthr);
         ma.xwait = xwait;
         ma.xto = xto;
         int pm = prof_begin("main_kernel", st);
-        e = launch_main(dt, p.NB, ma, dim3((unsigned)p.nwg, (unsigned)p.nbc), st);
+        e = launch_main(dt, p.NB, p.S, ma, dim3((unsigned)p.nwg, (unsigned)p.nbc), st);
         prof_end(pm, st);
         if (e != hipSuccess) return hip_fail(e, "main_kernel launch");
         mg.list_keys = list_keys; mg.list_cnt = list_cnt; mg.list_cap = p.list_cap;
@@ -551,7 +591,7 @@ static int run_exact(const ExactPlan& p, const TestHooks& hooks, const void* X, 
     // at xmax + r * (words per row), its threshold at xthr + r
     mg.xmax = p.xch ? (uint64_t*)(ws + p.off_xmax) : nullptr;
     mg.xthr = p.xch ? (uint64_t*)(ws + p.off_xthr) : nullptr;
-    mg.xmax_row = p.xch ? (p.large ? cdiv(p.num_tiles, p.tpw) * kLXchPerWg : (int64_t)p.nwg) : 0;
+    mg.xmax_row = p.xch ? (p.large ? cdiv(p.num_tiles, p.tpw) * kLXchPerWg : (int64_t)p.nwg * p.xper) : 0;
     mg.ties = 0;   // one encode's keys are distinct
     mg.V = V; mg.I = I;
     const int pg = prof_begin("merge_kernel", st);

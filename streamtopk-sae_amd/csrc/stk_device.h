@@ -353,22 +353,40 @@ __device__ __forceinline__ uint64_t compact_row(uint64_t* q, int n, uint64_t* sc
 
 // ---------------------------------------------------------------------------
 // TileStream: the score main loop with both operands staged in LDS.  A tile
-// is 32*WAVES latents x 32*NB rows and takes nds2 d-steps: the nds real ones
-// rounded up to even (a padding step loads a valid step again and skips its
-// MFMAs).
-//   W: each d-step's kTileF rows x 128 bytes are read with whole-line
-//      nontemporal loads (W is read once: no cache allocation), eight lanes
-//      per row step, two steps ahead in registers, and stored to a two-buffer
-//      LDS ring; each wave then reads its 32 rows in the MFMA layout.  Loads
-//      straight into the MFMA layout touch 32 rows per instruction, 32 bytes
-//      of each line, and stream W at ~6 TB/s; whole-line nontemporal loads
-//      reach ~7 TB/s.
+// is 32*WAVES/S latents x 32*NB rows; a step covers S 128-byte sub-steps of d.
+// A tile takes nds2 steps: the nds real ones rounded up to even (a padding
+// step loads a valid step again and skips its MFMAs).
+//   Split (S): the waves form S groups of WAVES / S; group q scores the tile's
+//      latents over sub-step q of every step, and the groups' partial sums are
+//      added in order before the epilogue (reduce).  Every step reads the same
+//      32 KiB of W whatever S, so S divides the steps of a tile and multiplies
+//      the tiles: a dictionary with fewer 256-latent tiles than CUs then
+//      spreads over more of them.  bf16, B = 32, d = 4096, F = 16384 (64 tiles
+//      of 64 steps, against 256 of 16): main_kernel 59.3 -> 31.3 us.
+//   W: each step's kTileF rows x S*128 bytes are read with whole-line loads
+//      (NT: nontemporal, see nontemporal_w), 8 S lanes per row, two steps
+//      ahead in registers, and stored to a two-buffer LDS ring; each wave then
+//      reads its 32 rows in the MFMA layout.  Loads straight into the MFMA
+//      layout touch 32 rows per instruction, 32 bytes of each line, and stream
+//      W at ~6 TB/s; whole-line nontemporal loads reach ~7 TB/s.
 //   X: the row block's 32*NB rows of the step, the same way with ordinary
 //      loads (every workgroup of the row block re-reads X from L2).
-// One barrier per d-step.  The loads of the next tile's first steps are in
-// flight across the epilogue.  Every load is unconditional (rows past F or B
-// and steps past the end are clamped to valid addresses; the scores they
-// produce are never selected).
+//   Rotation (rot): where a row is a multiple of 4 KiB, step s reads column
+//      step (s + 7 x) % nds, x the workgroup's place along W.  All workgroups
+//      start together, and at the same column their rows then fall on few
+//      memory channels: bf16, B = 1, d = 2048, F = 65536 68.4 us unrotated,
+//      47.7 us rotated (5.6 TB/s); F = 131072 124.6 and 85.9 us; at F = 2^18,
+//      where the workgroups drift apart, 163 us either way.  At 2 KiB rows it
+//      gained nothing.
+// The tile's rows of W and the row block's of X are buffer resources, rebuilt
+// per tile: rows past the range or past B, and the chunks past d of a partial
+// last step (an offset past every resource), read as zeros without a branch
+// or a mask, and a thread keeps one offset per operand.  bf16, B = 128,
+// d = 1000, F = 65536 (partial last step, rows no whole lines): main_kernel
+// 54.5 us with pointers, a branch for the last step and nontemporal loads,
+// 42.5 us so.
+// One barrier per step.  The loads of the next tile's first steps are in
+// flight across the epilogue.
 //
 // run() calls epi(t, acc, bias) after the last d-step of tile t and then
 // resets acc and waits for every outstanding memory operation: the epilogue
@@ -386,90 +404,100 @@ __device__ __forceinline__ uint64_t compact_row(uint64_t* q, int n, uint64_t* sc
 // add the products onto it); otherwise they start at zero and epi receives
 // the bias to add.
 // ---------------------------------------------------------------------------
-template <int DT, int NB, int WAVES>
+template <int DT, int NB, int WAVES, int S, bool NT>
 struct TileStream {
-    static constexpr int DS = Dt<DT>::DS;
+    static constexpr int DS = Dt<DT>::DS * S;                      // elements of d per step
     static constexpr int ES = Dt<DT>::esize;
     static constexpr int kThr = 64 * WAVES;
-    static constexpr int kTileF = 32 * WAVES;                      // latents per tile
-    static constexpr int kWChunks = kTileF * 8 / kThr;             // 16-byte W chunks per thread per step
-    static constexpr int kXTotal = 32 * NB * 8;                    // 16-byte X chunks per step
+    static constexpr int kLatWaves = WAVES / S;                    // waves across a tile's latents
+    static constexpr int kTileF = 32 * kLatWaves;                  // latents per tile
+    static constexpr int kRowChunks = 8 * S;                       // 16-byte chunks of a row per step
+    static constexpr int kWChunks = kTileF * kRowChunks / kThr;    // 16-byte W chunks per thread per step
+    static constexpr int kXTotal = 32 * NB * kRowChunks;           // 16-byte X chunks per step
     static constexpr int kXChunks = (kXTotal + kThr - 1) / kThr;   // per thread
-    static constexpr int kWBuf = kTileF * kXRowStride;             // bytes of one W ring buffer
-    static constexpr int kXBuf = 32 * NB * kXRowStride;            // bytes of one X ring buffer
+    static constexpr int kWBuf = S * kTileF * kXRowStride;         // bytes of one W ring buffer
+    static constexpr int kXBuf = S * 32 * NB * kXRowStride;        // bytes of one X ring buffer
     static constexpr int kRingBytes = 2 * kWBuf + 2 * kXBuf;
     static_assert(kXTotal % kThr == 0 || kXChunks == 1, "X chunk split");
-    static_assert(kTileF * 8 % kThr == 0, "W chunk split");
+    static_assert(kTileF * kRowChunks % kThr == 0, "W chunk split");
+    static_assert(kThr % kRowChunks == 0, "a thread's chunks share their place in the row");
+    static_assert(WAVES % S == 0 && S * NB <= 4, "ring size");
+    // the split waves' partial sums (before each epilogue) fit W ring buffer 1
+    static constexpr int kRedBytes = (WAVES - kLatWaves) * NB * 4096;
+    static_assert(kRedBytes <= kWBuf, "partial sums fit the idle ring buffer");
 
     static constexpr int kQE = 16 / ES;                            // elements per 16-byte chunk
 
     const float* bias;
-    int64_t F;
-    int64_t tile_begin;
+    int64_t F;                   // end of this workgroup's latents
+    int64_t f_begin;             // its first latent (tile t starts at f_begin + t * kTileF)
     int ntiles, nds, nds2;
-    int tail;                    // elements of d in the last d-step when it is partial, else 0
+    int tail;                    // elements of d in the last step when it is partial, else 0
+    int rot;                     // step s reads the columns of step (s + rot) % nds
     int tid, lane, wave, h, jl;
     const unsigned char* W;
     int64_t w_row_bytes;
 
-    // load cursor (uniform) and this thread's chunk pointers in the cursor's tile
+    // load cursor (uniform): the tile's rows and the row block as buffer
+    // resources (rows past the range or past B lie outside and read as zeros),
+    // this thread's offset of its first chunk in each
     int lt, ls;
-    const unsigned char* lw[kWChunks];
-    const unsigned char* lx[kXChunks];
-    bool xok[kXChunks];
+    __amdgpu_buffer_rsrc_t wres, xres;
+    int woff, xoff;
+    int toff;                    // added in the partial last step: out of range for a chunk past d
 
-    __device__ __forceinline__ void init_x(const unsigned char* X, int64_t B, int64_t b0, int64_t d)
+    // d, the row stride and the alignment of W decide the steps, the partial
+    // last step, the load kind and the rotation; `x` is the workgroup's place
+    // along W.
+    __device__ __forceinline__ void init_steps(int64_t d, int x)
     {
-#pragma unroll
-        for (int p = 0; p < kXChunks; ++p) {
-            const int c = tid + kThr * p;
-            const int row = (c >> 3) % (32 * NB), c16 = c & 7;
-            int64_t r = b0 + row;
-            r = (r < B) ? r : B - 1;
-            lx[p] = X + (r * d) * ES + c16 * 16;
-            xok[p] = c < kXTotal;
-        }
+        nds = (int)((d + DS - 1) / DS);
+        tail = (int)(d % DS);
+        nds2 = (nds + 1) / 2 * 2;
+        w_row_bytes = d * ES;
+        rot = (w_row_bytes & 4095) == 0 ? (int)(((unsigned)x * 7u) % (unsigned)nds) : 0;
+    }
+
+    __device__ __forceinline__ int col(int s) const   // column step of step s (s >= nds: any valid one)
+    {
+        const int c = (s < nds ? s : nds - 1) + rot;
+        return c >= nds ? c - nds : c;
+    }
+
+    static constexpr int kOut = 0x40000000;   // an offset beyond every resource (tiles and row blocks: at most 4 MiB)
+
+    __device__ __forceinline__ void init_x(const unsigned char* X, int64_t B, int64_t b0)
+    {
+        const int64_t nrows = B - b0 < 32 * NB ? B - b0 : 32 * NB;
+        xres = make_rsrc(X + b0 * w_row_bytes, nrows * w_row_bytes);
+        const int off = tid / kRowChunks * (int)w_row_bytes + tid % kRowChunks * 16;
+        woff = off;
+        xoff = tid < kXTotal ? off : kOut;
+        toff = (tid % kRowChunks) * kQE < tail ? 0 : kOut;
     }
 
     __device__ __forceinline__ void set_rows(int t)
     {
-        const int64_t tile = tile_begin + (t < ntiles ? t : ntiles - 1);
-#pragma unroll
-        for (int p = 0; p < kWChunks; ++p) {
-            const int c = tid + kThr * p;
-            int64_t f = tile * kTileF + (c >> 3);
-            f = (f < F) ? f : F - 1;
-            lw[p] = W + f * w_row_bytes + (c & 7) * 16;
-        }
+        const int64_t f0 = f_begin + (int64_t)t * kTileF;
+        const int64_t n = F - f0 < kTileF ? F - f0 : kTileF;
+        wres = make_rsrc(W + f0 * w_row_bytes, n * w_row_bytes);
     }
 
+    // Loads of the cursor's step (past the last tile: any valid one), in
+    // ascending address order; a thread's chunks lie kThr / kRowChunks rows
+    // apart and share their place in the row.
     __device__ __forceinline__ void issue(u32x4 (&xr)[kXChunks], u32x4 (&wr)[kWChunks])
     {
-        const int s = (lt >= ntiles || ls >= nds) ? nds - 1 : ls;
-        const int64_t so = (int64_t)s * kStepBytes;
-        if (tail != 0 && s == nds - 1) {
-            // partial last step: a chunk past d reads the step's first chunk
-            // (in bounds: the step starts below d) and is zeroed
+        const int s = col(lt < ntiles ? ls : nds);
+        const int so = __builtin_amdgcn_readfirstlane(s * (S * kStepBytes));
+        const int to = (tail != 0 && s == nds - 1) ? toff : 0;
 #pragma unroll
-            for (int p = 0; p < kXChunks; ++p) {
-                const int c8 = (tid + kThr * p) & 7;
-                const bool ok = c8 * kQE < tail;
-                const u32x4 v = *(const u32x4*)(lx[p] + so - (ok ? 0 : c8 * 16));
-                xr[p] = ok ? v : u32x4{0u, 0u, 0u, 0u};
-            }
+        for (int p = 0; p < kXChunks; ++p)
+            xr[p] = __builtin_amdgcn_raw_buffer_load_b128(xres, xoff + to, so + p * (kThr / kRowChunks) * (int)w_row_bytes, 0);
 #pragma unroll
-            for (int p = 0; p < kWChunks; ++p) {
-                const int c8 = (tid + kThr * p) & 7;
-                const bool ok = c8 * kQE < tail;
-                const u32x4 v = __builtin_nontemporal_load((const u32x4*)(lw[p] + so - (ok ? 0 : c8 * 16)));
-                wr[p] = ok ? v : u32x4{0u, 0u, 0u, 0u};
-            }
-        } else {
-#pragma unroll
-            for (int p = 0; p < kXChunks; ++p) xr[p] = *(const u32x4*)(lx[p] + so);
-#pragma unroll
-            for (int p = 0; p < kWChunks; ++p) wr[p] = __builtin_nontemporal_load((const u32x4*)(lw[p] + so));
-        }
+        for (int p = 0; p < kWChunks; ++p)
+            wr[p] = __builtin_amdgcn_raw_buffer_load_b128(wres, woff + to, so + p * (kThr / kRowChunks) * (int)w_row_bytes,
+                                                          NT ? 2 : 0);
         if (lt < ntiles && ++ls == nds2) {
             ls = 0;
             ++lt;
@@ -477,23 +505,29 @@ struct TileStream {
         }
     }
 
-    __device__ __forceinline__ void store(const u32x4 (&xr)[kXChunks], const u32x4 (&wr)[kWChunks],
-                                          unsigned char* xs, unsigned char* wsb) const
+    // LDS offset of a thread's chunk p in a ring buffer of `rows` rows per
+    // 128-byte sub-step
+    __device__ __forceinline__ int ring_off(int p, int rows) const
+    {
+        const int c = tid + kThr * p;
+        return (((c % kRowChunks) >> 3) * rows + c / kRowChunks) * kXRowStride + (c & 7) * 16;
+    }
+
+    __device__ __forceinline__ void store(const u32x4 (&xr)[kXChunks], const u32x4 (&wr)[kWChunks], unsigned char* xs,
+                                          unsigned char* wsb) const
     {
 #pragma unroll
-        for (int p = 0; p < kWChunks; ++p) {
-            const int c = tid + kThr * p;
-            *(u32x4*)(wsb + (c >> 3) * kXRowStride + (c & 7) * 16) = wr[p];
-        }
+        for (int p = 0; p < kWChunks; ++p) *(u32x4*)(wsb + ring_off(p, kTileF)) = wr[p];
 #pragma unroll
-        for (int p = 0; p < kXChunks; ++p) {
-            const int c = tid + kThr * p;
-            if (kXTotal % kThr == 0 || xok[p]) *(u32x4*)(xs + (c >> 3) * kXRowStride + (c & 7) * 16) = xr[p];
-        }
+        for (int p = 0; p < kXChunks; ++p)
+            if (kXTotal % kThr == 0 || tid < kXTotal) *(u32x4*)(xs + ring_off(p, 32 * NB)) = xr[p];
     }
 
     __device__ __forceinline__ void compute(f32x16 (&acc)[NB], const unsigned char* xs, const unsigned char* wsb) const
     {
+        // wave -> sub-step wave / kLatWaves, latents 32 (wave % kLatWaves) ..:
+        // its W rows are ring rows 32 wave ..
+        const unsigned char* xw = xs + (S > 1 ? wave / kLatWaves * (32 * NB) : 0) * kXRowStride;
         u32x4 w[4];
 #pragma unroll
         for (int q = 0; q < 4; ++q) w[q] = *(const u32x4*)(wsb + (wave * 32 + jl) * kXRowStride + h * 64 + q * 16);
@@ -506,7 +540,7 @@ struct TileStream {
             for (int n = 0; n < NP; ++n)
 #pragma unroll
                 for (int q = 0; q < 4; ++q)
-                    bx[n][q] = *(const u32x4*)(xs + (32 * (n0 + n) + jl) * kXRowStride + h * 64 + q * 16);
+                    bx[n][q] = *(const u32x4*)(xw + (32 * (n0 + n) + jl) * kXRowStride + h * 64 + q * 16);
 #pragma unroll
             for (int q = 0; q < 4; ++q)
 #pragma unroll
@@ -516,7 +550,7 @@ struct TileStream {
 
     __device__ __forceinline__ void bias_load(float (&bn)[kTileF / 64], int t) const
     {
-        const int64_t f0 = (tile_begin + t) * kTileF + lane * (kTileF / 64);
+        const int64_t f0 = f_begin + (int64_t)t * kTileF + lane * (kTileF / 64);
 #pragma unroll
         for (int e = 0; e < kTileF / 64; ++e) {
             const int64_t f = f0 + e;
@@ -544,7 +578,7 @@ struct TileStream {
 
     __device__ __forceinline__ void acc_reset(f32x16 (&acc)[NB], const float* bias_buf, bool from_bias) const
     {
-        if (from_bias) {
+        if (from_bias && (S == 1 || wave < kLatWaves)) {
             float bv[16];
             bias_read(bv, bias_buf);
 #pragma unroll
@@ -556,6 +590,37 @@ struct TileStream {
             for (int n = 0; n < NB; ++n)
 #pragma unroll
                 for (int r = 0; r < 16; ++r) acc[n][r] = 0.f;
+        }
+    }
+
+    // S > 1: the sub-step waves' partial sums, added in sub-step order to the
+    // waves of sub-step 0 through W ring buffer 1 (idle; its next writer runs
+    // after a barrier of the epilogue).
+    __device__ __forceinline__ void reduce(f32x16 (&acc)[NB], unsigned char* red) const
+    {
+        if constexpr (S > 1) {
+            f32x4* mine = (f32x4*)red + lane;
+            if (wave >= kLatWaves) {
+#pragma unroll
+                for (int n = 0; n < NB; ++n)
+#pragma unroll
+                    for (int g = 0; g < 4; ++g)
+                        mine[(((wave - kLatWaves) * NB + n) * 4 + g) * 64] =
+                            f32x4{acc[n][4 * g], acc[n][4 * g + 1], acc[n][4 * g + 2], acc[n][4 * g + 3]};
+            }
+            __syncthreads();
+            if (wave < kLatWaves) {
+#pragma unroll
+                for (int q = 0; q < S - 1; ++q)
+#pragma unroll
+                    for (int n = 0; n < NB; ++n)
+#pragma unroll
+                        for (int g = 0; g < 4; ++g) {
+                            const f32x4 v = mine[(((q * kLatWaves + wave) * NB + n) * 4 + g) * 64];
+#pragma unroll
+                            for (int e = 0; e < 4; ++e) acc[n][4 * g + e] += v[e];
+                        }
+            }
         }
     }
 
@@ -598,6 +663,7 @@ struct TileStream {
                 if (wave == 0) bias_store(bn, bnext);
                 __syncthreads();
             }
+            reduce(acc, ws1);
             float bv[16];
             if (!kBiasInit) bias_read(bv, bias_lds + (t & 1) * kTileF);
             epi(t, acc, bv);

@@ -37,6 +37,7 @@ constexpr int kMainWaves = 8;        // wavefronts per main_kernel workgroup (2 
 constexpr int kMainThreads = 64 * kMainWaves;
 constexpr int kTileLatents = 32 * kMainWaves;   // latents per main_kernel tile
 constexpr int kApproxGroup = 128;    // latent group of the approximate variant
+constexpr int kRangeUnit = 16;       // main_kernel's workgroups share the latents in units of this many
 constexpr int kGroupTile = 256;      // latents per group_kernel tile (two groups)
 constexpr int kSampleTarget = 4096;  // sampled latents that seed the thresholds
 constexpr int kSampleLarge = 8192;   //   (large batches with F >= kSampleLargeMinF)
@@ -67,7 +68,6 @@ struct MainArgs {
     const float* bias;
     int64_t B, d, F;
     int k, cap;
-    int64_t num_tiles, tiles_per_wg;
     const uint64_t* thr0;        // per-row starting threshold keys, or null
     int sampled;                 // non-zero: the sampled latents (is_sampled) were
     int samp_log2, samp_blocks;  //   scored by the sample pass and are skipped here
@@ -87,7 +87,8 @@ struct MainArgs {
     // before its first epilogue filters anything.  Each word: the call's tag
     // tag << 32 | a score image (ordered_u32).
     int xch;
-    uint64_t* xmax;              // [nbc][32*NB][gridDim.x] each workgroup's row maxima
+    int xper;                    // maxima per row and workgroup (each over the latents of 8 / S / xper waves)
+    uint64_t* xmax;              // [nbc][32*NB][gridDim.x * xper] each workgroup's row maxima
     uint64_t* xthr;              // [nbc][32*NB] row thresholds (owner x: rows x, x + gridDim.x, ...)
     int64_t xwait;               // s_memrealtime ticks a wave polls for words before going
                                  //   on without the exchanged thresholds (threshold 0)
@@ -312,12 +313,24 @@ struct CandArgs {                // approximate variant, top-k over the candidat
     int32_t* I;
 };
 
-size_t main_lds_bytes(int NB, int cap, int lq);
-int main_lds_queue(int NB, int k);
+// Whether the streaming kernels below 512 rows read W with nontemporal loads:
+// when one row block reads it (each line is then used once) and its rows are
+// whole 128-byte lines.  Other rows share their boundary lines between
+// d-steps, which nontemporal loads fetched from memory twice, and several row
+// blocks share every line through L2.  Measured, bf16, nontemporal / cached:
+// B = 1, F = 2^18: d = 2048 164 / 182 us, d = 2056 261 / 196 us; B = 200 (two
+// row blocks), d = 960, F = 2^16: 57.7 / 51.5 us.
+inline bool nontemporal_w(const void* W, int64_t row_bytes, int64_t row_blocks)
+{
+    return row_blocks == 1 && (((uintptr_t)W | (uintptr_t)row_bytes) & (kStepBytes - 1)) == 0;
+}
+
+size_t main_lds_bytes(int NB, int S, int cap, int lq);
+int main_lds_queue(int NB, int S, int k);
 size_t mainl_lds_bytes(int cap);
 size_t group_lds_bytes(int NB);
 
-hipError_t launch_main(int dt, int NB, const MainArgs& a, dim3 grid, hipStream_t st);
+hipError_t launch_main(int dt, int NB, int S, const MainArgs& a, dim3 grid, hipStream_t st);
 hipError_t launch_mainl(int dt, const MainLArgs& a, int grid, hipStream_t st);
 hipError_t launch_mainl_sample(int dt, const MainLArgs& a, int grid, hipStream_t st);
 hipError_t launch_sample(int dt, int NB, const SampleArgs& a, dim3 grid, hipStream_t st);
@@ -325,6 +338,7 @@ hipError_t launch_thr(const ThrArgs& a, int64_t rows, hipStream_t st);
 hipError_t launch_merge(const MergeArgs& a, int64_t rows, hipStream_t st);
 hipError_t launch_pack(const PackArgs& a, int64_t rows, hipStream_t st);
 hipError_t launch_group(int dt, int NB, const GroupArgs& a, dim3 grid, hipStream_t st);
+hipError_t launch_group_cached(int dt, int NB, const GroupArgs& a, dim3 grid, hipStream_t st);
 hipError_t launch_cand(const CandArgs& a, int64_t rows, hipStream_t st);
 hipError_t launch_read_probe(const void* buf, int64_t n16, uint32_t* sink, int ncu, hipStream_t st);
 // Zero-fills `bytes` (a multiple of 16) at 16-byte aligned `p` with a kernel (no memset node).

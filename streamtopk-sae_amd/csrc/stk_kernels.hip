@@ -162,11 +162,12 @@ __device__ __forceinline__ void flush_rows(int* cnt, int* gcnt, uint64_t* thr, c
 // affected thresholds at 0, which accepts every score: the result stays
 // exact, the call only slower.  scr: 8 * BT LDS words, free while the
 // epilogue runs.
-template <int NB>
+template <int NB, int LW>
 __device__ __forceinline__ void xch_thresholds(const MainArgs& a, const f32x16 (&ac)[NB], uint32_t vmask,
                                                uint64_t* thr, uint32_t* scr, int64_t b0, int tid, uint32_t tag)
 {
     constexpr int BT = 32 * NB;
+    const int xper = a.xper, nw = (int)gridDim.x * xper;   // maxima per workgroup and row, per row
     const int lane = tid & 63, wave = tid >> 6, h = lane >> 5, jl = lane & 31;
     const int nwg = (int)gridDim.x, x = (int)blockIdx.x;
     const int nrows = (int)(a.B - b0 < BT ? a.B - b0 : BT);
@@ -175,7 +176,7 @@ __device__ __forceinline__ void xch_thresholds(const MainArgs& a, const f32x16 (
     // from it is hoisted out of the tile loop (kept live, it would spill)
     int64_t yb = blockIdx.y;
     asm volatile("" : "+s"(yb));
-    uint64_t* xmax = a.xmax + yb * BT * nwg;   // [BT][nwg]
+    uint64_t* xmax = a.xmax + yb * BT * nw;    // [BT][nw]
     uint64_t* xthr = a.xthr + yb * BT;         // [BT]
 
 #pragma unroll
@@ -188,23 +189,24 @@ __device__ __forceinline__ void xch_thresholds(const MainArgs& a, const f32x16 (
         if (h == 0) scr[wave * BT + 32 * n + jl] = q > o ? q : o;
     }
     __syncthreads();
-    if (tid < nrows) {
-        uint32_t m = scr[tid];
-#pragma unroll
-        for (int w = 1; w < kMainWaves; ++w) {
-            const uint32_t o = scr[w * BT + tid];
+    const int wpp = LW / xper;   // waves per published maximum
+    for (int i = tid; i < BT * xper; i += kMainThreads) {
+        const int r = i % BT, part = i / BT;
+        uint32_t m = 0u;
+        for (int w = part * wpp; w < (part + 1) * wpp; ++w) {
+            const uint32_t o = scr[w * BT + r];
             m = o > m ? o : m;
         }
-        xch_put(xmax + (int64_t)tid * nwg + x, tag, m);
+        if (r < nrows) xch_put(xmax + (int64_t)r * nw + x * xper + part, tag, m);
     }
 
     const int row = x + wave * nwg;
     if (x < nown && row < nrows) {
         uint32_t v[4];
         uint32_t T = 0;
-        const int quorum = (3 * nwg + 3) / 4;
+        const int quorum = (3 * nw + 3) / 4;
         const int need = a.k > quorum ? a.k : quorum;
-        const int got = xch_poll<4>(xmax + (int64_t)row * nwg, nwg, need, tag, a.xwait, lane, v);
+        const int got = xch_poll<4>(xmax + (int64_t)row * nw, nw, need, tag, a.xwait, lane, v);
         // any k arrived maxima bound the k-th score, a quorum or not
         if (got >= a.k) T = xch_kth<4>(v, a.k);
         if (got < need && lane == 0 && a.xwait > 0) atomicAdd(a.xto, 1u);
@@ -225,20 +227,20 @@ __device__ __forceinline__ void xch_thresholds(const MainArgs& a, const f32x16 (
     __syncthreads();
 }
 
-template <int DT, int NB>
+template <int DT, int NB, int S, bool NT>
 __global__ __launch_bounds__(kMainThreads, 2) void main_kernel(MainArgs a)
 {
     constexpr int BT = 32 * NB;
     constexpr int WAVES = kMainWaves;
     constexpr int R = BT / WAVES;   // rows each wave spills and flushes
-    using TS = TileStream<DT, NB, WAVES>;
+    using TS = TileStream<DT, NB, WAVES, S, NT>;
     extern __shared__ __align__(16) unsigned char smem[];
     const int cap = a.cap, lq = a.lq;
     uint64_t* thr = (uint64_t*)(smem + TS::kRingBytes);          // [BT] row threshold keys
     int* cnt = (int*)(thr + BT);                                   // [BT] LDS queue fill counts
     int* gcnt = cnt + BT;                                          // [BT] global segment fill counts
-    float* bias_lds = (float*)(gcnt + BT);                         // [2][kTileLatents]
-    uint64_t* lqk = (uint64_t*)(bias_lds + 2 * kTileLatents);      // [BT][lq] LDS queues
+    float* bias_lds = (float*)(gcnt + BT);                         // [2][TS::kTileF]
+    uint64_t* lqk = (uint64_t*)(bias_lds + 2 * TS::kTileF);         // [BT][lq] LDS queues
     uint64_t* cscr = lqk + BT * lq;                                // [WAVES][cap] compaction scratch
     uint32_t* vote = (uint32_t*)(cscr + WAVES * cap);              // [2][WAVES] block_any slots (cap even: 16-byte aligned)
     uint32_t vpar = 0;
@@ -246,7 +248,7 @@ __global__ __launch_bounds__(kMainThreads, 2) void main_kernel(MainArgs a)
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int h = lane >> 5, jl = lane & 31;
     const int64_t b0 = (int64_t)blockIdx.y * BT;
-    const int64_t B = a.B, F = a.F;
+    const int64_t B = a.B;
     const int k = a.k;
     // this call's tag: the workspace's epoch (advanced by the previous call's
     // merge) + 1, recorded for this call's merge after the first tile (the
@@ -264,23 +266,24 @@ __global__ __launch_bounds__(kMainThreads, 2) void main_kernel(MainArgs a)
 
     TS ts;
     ts.W = (const unsigned char*)a.W;
-    ts.w_row_bytes = a.d * Dt<DT>::esize;
     ts.bias = a.bias;
-    ts.F = F;
-    ts.tile_begin = (int64_t)blockIdx.x * a.tiles_per_wg;
+    // latents [f_begin, F): the workgroups' ranges differ by at most
+    // kRangeUnit latents, the last tile of a range may be partial
     {
-        const int64_t t1 = ts.tile_begin + a.tiles_per_wg;
-        ts.ntiles = (int)((t1 < a.num_tiles ? t1 : a.num_tiles) - ts.tile_begin);
+        const int64_t nu = (a.F + kRangeUnit - 1) / kRangeUnit, nx = gridDim.x, x = blockIdx.x;
+        const int64_t f1 = (x + 1) * nu / nx * kRangeUnit;
+        ts.f_begin = x * nu / nx * kRangeUnit;
+        ts.F = f1 < a.F ? f1 : a.F;
     }
-    ts.nds = (int)((a.d + Dt<DT>::DS - 1) / Dt<DT>::DS);
-    ts.tail = (int)(a.d % Dt<DT>::DS);
-    ts.nds2 = (ts.nds + 1) / 2 * 2;
+    const int64_t F = ts.F;
+    ts.ntiles = (int)((F - ts.f_begin + TS::kTileF - 1) / TS::kTileF);
+    ts.init_steps(a.d, (int)blockIdx.x);
     ts.tid = tid;
     ts.lane = lane;
     ts.wave = wave;
     ts.h = h;
     ts.jl = jl;
-    ts.init_x((const unsigned char*)a.X, B, b0, a.d);
+    ts.init_x((const unsigned char*)a.X, B, b0);
 
     f32x16 acc[NB];
     // the accumulators start at the bias: ac holds the scores at the epilogue
@@ -292,12 +295,12 @@ __global__ __launch_bounds__(kMainThreads, 2) void main_kernel(MainArgs a)
             if (tid == 0 && blockIdx.x == 0 && blockIdx.y == 0) clear_stale_err(a.err, tag);
         }
         // latent of accumulator register r of this lane: fl + 8*(r/4) + r%4
-        const int64_t tile0 = (ts.tile_begin + t) * (int64_t)kTileLatents;
+        const int64_t tile0 = ts.f_begin + t * (int64_t)TS::kTileF;
         const int64_t fl = tile0 + wave * 32 + h * 4;
-        // latents past F or in the sample are never candidates here
-        uint32_t vmask = 0xFFFFu;
-        if (tile0 + kTileLatents > F || (a.sampled && (is_sampled(tile0, a.samp_log2, a.samp_blocks) ||
-                                                       is_sampled(tile0 + kTileLatents - 1, a.samp_log2, a.samp_blocks)))) {
+        // latents past the range or in the sample are never candidates here;
+        // the scores are with the waves of sub-step 0
+        uint32_t vmask = wave < TS::kLatWaves ? 0xFFFFu : 0u;
+        if (wave < TS::kLatWaves && (tile0 + TS::kTileF > F || a.sampled)) {
             vmask = 0;
 #pragma unroll
             for (int r = 0; r < 16; ++r) {
@@ -306,7 +309,9 @@ __global__ __launch_bounds__(kMainThreads, 2) void main_kernel(MainArgs a)
                 vmask |= ok ? (1u << r) : 0u;
             }
         }
-        if (a.xch && t == 0) xch_thresholds<NB>(a, ac, vmask, thr, (uint32_t*)(smem + TS::kWBuf), b0, tid, tag);
+        if (a.xch && t == 0) 
+            xch_thresholds<NB, TS::kLatWaves>(a, ac, vmask, thr, (uint32_t*)(smem + TS::kWBuf + TS::kRedBytes), b0, tid,
+                                              tag);
         // ---- scores not below the row threshold ----
         // The float test keeps every score whose key beats the threshold key
         // (and possibly a few equal to its value: harmless extra candidates).
@@ -1022,43 +1027,53 @@ __global__ __launch_bounds__(kProbeThreads) void read_probe_kernel(const u32x4* 
 // ---------------------------------------------------------------------------
 // Host-side launch helpers
 // ---------------------------------------------------------------------------
-size_t main_lds_bytes(int NB, int cap, int lq)
+size_t main_lds_bytes(int NB, int S, int cap, int lq)
 {
     const size_t BT = 32 * (size_t)NB;
-    const size_t rings = 2 * (size_t)kTileLatents * kXRowStride + 2 * BT * kXRowStride;   // TileStream rings
-    return rings + BT * 8 + BT * 8 + 2 * kTileLatents * 4 + BT * (size_t)lq * 8 + (size_t)kMainWaves * cap * 8 +
+    const size_t rings = 2 * (size_t)kTileLatents * kXRowStride + 2 * S * BT * kXRowStride;   // TileStream rings
+    return rings + BT * 8 + BT * 8 + 2 * (kTileLatents / S) * 4 + BT * (size_t)lq * 8 + (size_t)kMainWaves * cap * 8 +
            2 * kMainWaves * sizeof(uint32_t);
 }
 
 // LDS queue keys per row: the most (even, at most 64) whose LDS use, with
 // global segments of cap = k + lq keys, fits 159 KiB of the workgroup's 160.
-int main_lds_queue(int NB, int k)
+int main_lds_queue(int NB, int S, int k)
 {
     for (int lq = 64; lq >= 2; lq -= 2) {
         const int cap = (k + lq + 1) & ~1;
-        if (main_lds_bytes(NB, cap, lq) <= 159 * 1024) return lq;
+        if (main_lds_bytes(NB, S, cap, lq) <= 159 * 1024) return lq;
     }
     return 0;
 }
 
-template <int DT, int NB>
+template <int DT, int NB, int S, bool NT>
 static hipError_t launch_main_t(const MainArgs& a, dim3 grid, hipStream_t st)
 {
-    const size_t lds = main_lds_bytes(NB, a.cap, a.lq);
-    auto kern = main_kernel<DT, NB>;
+    const size_t lds = main_lds_bytes(NB, S, a.cap, a.lq);
+    auto kern = main_kernel<DT, NB, S, NT>;
     hipError_t e = ensure_lds((const void*)kern, lds);
     if (e != hipSuccess) return e;
     launch(kern, grid, dim3(kMainThreads), lds, st, a);
     return hipGetLastError();
 }
 
-hipError_t launch_main(int dt, int NB, const MainArgs& a, dim3 grid, hipStream_t st)
+template <int DT, bool NT>
+static hipError_t launch_main_s(int NB, int S, const MainArgs& a, dim3 grid, hipStream_t st)
 {
-#define STK_CASE(DTV, NBV) \
-    if (dt == DTV && NB == NBV) return launch_main_t<DTV, NBV>(a, grid, st);
-    STK_CASE(DT_BF16, 1) STK_CASE(DT_BF16, 2) STK_CASE(DT_BF16, 4)
-    STK_CASE(DT_F16, 1) STK_CASE(DT_F16, 2) STK_CASE(DT_F16, 4)
-    STK_CASE(DT_F32, 1) STK_CASE(DT_F32, 2) STK_CASE(DT_F32, 4)
+#define STK_CASE(NBV, SV) \
+    if (NB == NBV && S == SV) return launch_main_t<DT, NBV, SV, NT>(a, grid, st);
+    STK_CASE(1, 1) STK_CASE(2, 1) STK_CASE(4, 1)
+    STK_CASE(1, 2) STK_CASE(2, 2) STK_CASE(1, 4)
+#undef STK_CASE
+    return hipErrorInvalidValue;
+}
+
+hipError_t launch_main(int dt, int NB, int S, const MainArgs& a, dim3 grid, hipStream_t st)
+{
+    const bool nt = nontemporal_w(a.W, a.d * (dt == DT_F32 ? 4 : 2), grid.y);
+#define STK_CASE(DTV) \
+    if (dt == DTV) return nt ? launch_main_s<DTV, true>(NB, S, a, grid, st) : launch_main_s<DTV, false>(NB, S, a, grid, st);
+    STK_CASE(DT_BF16) STK_CASE(DT_F16) STK_CASE(DT_F32)
 #undef STK_CASE
     return hipErrorInvalidValue;
 }
