@@ -201,7 +201,7 @@ static ExactPlan make_exact_plan(int64_t B, int64_t d, int64_t F, int64_t k, int
 {
     ExactPlan p;
     p.num_tiles = cdiv(F, kTileLatents);
-    p.large = B >= kLargeMinB;
+    p.large = B >= (dtype == STK_DTYPE_F32 ? kLargeMinBF32 : kLargeMinB);
     p.lq = 0;
     p.S = 1;
     p.xper = 1;
@@ -271,13 +271,14 @@ static ExactPlan make_exact_plan(int64_t B, int64_t d, int64_t F, int64_t k, int
     // m = 64 above) or from a sample pass of nsamp latents (whose k-th is the
     // threshold).  A latent passes the exchange's threshold with probability
     // about -ln(1 - k / n) / m and the sample's about k / nsamp.  The exchange
-    // is taken when it passes at most as many (up to twice as many below 512
-    // rows with one maximum per workgroup, where it also saves the two launches
-    // of the sample and threshold passes, a larger share of the call); it needs n > k (n = k is the
-    // minimum of all maxima) and, below 512 rows, at least kXchMinWg
-    // workgroups.  Measured (B = 512-2048, d = 2048-4096, k = 64-128): the
+    // is taken when it passes at most as many (up to twice as many with one
+    // maximum per workgroup of main_kernel, where it also saves the two launches
+    // of the sample and threshold passes, a larger share of the call); it needs
+    // n > k (n = k is the minimum of all maxima) and, for main_kernel, at least
+    // kXchMinWg workgroups.  Measured (B = 512-2048, d = 2048-4096, k = 64-128): the
     // exchange was 3-8 % faster where it passes fewer latents, 1-4 % slower
-    // where it passes ~1.4x as many, and up to 2x slower at n = k.
+    // where it passes ~1.4x as many, and up to 2x slower at n = k; fp32, B = 1500,
+    // k = 128, 1.4x as many: 1483 us against 1109 with the sample pass.
     // (The no_xch test hook selects the sample pass.)
     const int samp_n = (p.large && F >= kSampleLargeMinF) ? kSampleLarge : kSampleTarget;
     {
@@ -340,7 +341,7 @@ static ExactPlan make_exact_plan(int64_t B, int64_t d, int64_t F, int64_t k, int
         // maxima over 256 latents each: a latent passes with probability
         // about -ln(1 - k / nwg) / 256, so a workgroup expects
         // -ln(1 - k / nwg) * tpw survivors per row.
-        const int lq_max = main_lds_queue(p.NB, p.S, (int)k);
+        const int lq_max = main_lds_queue(dtype, p.NB, p.S, (int)k);
         int lq = lq_max;
         p.expect_seg = p.cap;
         if (p.sample || p.xch) {
@@ -581,6 +582,9 @@ static int run_exact(const ExactPlan& p, const TestHooks& hooks, const void* X, 
         // to ~12, of 48 up to ~24, else of 64
         const int64_t per_seg = p.expect_seg;
         mg.spec = per_seg <= 3 ? 6 : per_seg <= 12 ? 3 : per_seg <= 24 ? 4 : 5;
+        // many rows (fp32): the merges of which four rows fit a CU, as after
+        // mainl_kernel (1024 rows of 32 segments: 43.7 us with 512 threads a row)
+        if (B >= kLargeMinB) mg.spec = p.head_span == 0 ? 8 : 0;
     }
     mg.k = (int)k;
     mg.f_offset = (int32_t)f_offset;

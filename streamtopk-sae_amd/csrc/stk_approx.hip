@@ -19,11 +19,11 @@
 
 namespace stk {
 
-size_t group_lds_bytes(int NB)
+size_t group_lds_bytes(int dt, int NB)
 {
-    const size_t rings = 2 * (size_t)kGroupTile * kXRowStride + 2 * 32 * (size_t)NB * kXRowStride;
-    return rings + 2 * kGroupTile * sizeof(float) + 32 * (size_t)kOrdStride * sizeof(uint32_t) +
-           32 * (size_t)NB * kHeadSlots * sizeof(uint64_t);
+    const size_t xs = dt == DT_F32 ? kXSplitStride : kXRowStride;
+    const size_t rings = 2 * (size_t)kGroupTile * kXRowStride + 2 * 32 * (size_t)NB * xs;
+    return rings + 2 * kGroupTile * sizeof(float) + 32 * (size_t)NB * kHeadSlots * sizeof(uint64_t);
 }
 
 template <int DT, int NB, int C>

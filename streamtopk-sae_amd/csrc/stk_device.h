@@ -25,10 +25,13 @@
 
 namespace stk {
 
+typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef float f32x2 __attribute__((ext_vector_type(2)));
 typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
+typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 typedef uint64_t u64x2 __attribute__((ext_vector_type(2)));
 
@@ -38,6 +41,7 @@ constexpr int kWaves = 4;            // wavefronts per workgroup
 constexpr int kThreads = 64 * kWaves;
 constexpr int kStepBytes = 128;      // bytes of one W/X row per d-step
 constexpr int kXRowStride = 144;     // LDS bytes per staged X row (128 + 16 pad)
+constexpr int kXSplitStride = 208;   // the same for fp32 X, as bf16 parts (3 * 64 + 16 pad)
 
 template <int DT> struct Dt;
 template <> struct Dt<DT_BF16> { static constexpr int esize = 2; static constexpr int DS = 64; };
@@ -268,6 +272,33 @@ __device__ __forceinline__ void mfma_quad<DT_F32>(f32x16& acc, u32x4 a, u32x4 b)
 }
 
 // ---------------------------------------------------------------------------
+// fp32 operands on the bf16 matrix cores.  A finite fp32 value is the sum of
+// three bf16 values, v = v1 + v2 + v3: each is the rest so far rounded to
+// nearest (8 significant bits, and the remainders are exact), so 24 bits are
+// covered.  Of the nine products of two split values the six of weight 2^-16
+// and more are formed (v1 w1, v1 w2, v2 w1, v1 w3, v2 w2, v3 w1), each exact
+// in fp32 and accumulated in fp32; the three left out are below 2^-24 of
+// v w each.  Six v_mfma_f32_32x32x16_bf16 take 192 cycles for what eight
+// v_mfma_f32_32x32x2_f32 take 512.  The splits exist for normal, finite
+// values: TileStream::fix_up recomputes scores that may have met others.
+// ---------------------------------------------------------------------------
+__device__ __forceinline__ uint32_t pk_bf16(float a, float b)
+{
+    return __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2){a, b}, bf16x2));
+}
+
+// The three bf16 parts of a and b, packed (a in the low halves).
+__device__ __forceinline__ void split3(float a, float b, uint32_t (&p)[3])
+{
+#pragma unroll
+    for (int i = 0; i < 3; ++i) {
+        p[i] = pk_bf16(a, b);
+        a -= __uint_as_float(p[i] << 16);
+        b -= __uint_as_float(p[i] & 0xFFFF0000u);
+    }
+}
+
+// ---------------------------------------------------------------------------
 // Compacts the queue segments (in global memory) of this wave's rows that are
 // full to their top-k: rows wave*R .. wave*R + R - 1 (R <= 64), segment of
 // row r at qrow(r), cap keys; cnt and thr in LDS.  Segment keys are read
@@ -355,7 +386,7 @@ __device__ __forceinline__ uint64_t compact_row(uint64_t* q, int n, uint64_t* sc
 // TileStream: the score main loop with both operands staged in LDS.  A tile
 // is 32*WAVES/S latents x 32*NB rows; a step covers S 128-byte sub-steps of d.
 // A tile takes nds2 steps: the nds real ones rounded up to even (a padding
-// step loads a valid step again and skips its MFMAs).
+// step reads zeros).
 //   Split (S): the waves form S groups of WAVES / S; group q scores the tile's
 //      latents over sub-step q of every step, and the groups' partial sums are
 //      added in order before the epilogue (reduce).  Every step reads the same
@@ -416,7 +447,11 @@ struct TileStream {
     static constexpr int kXTotal = 32 * NB * kRowChunks;           // 16-byte X chunks per step
     static constexpr int kXChunks = (kXTotal + kThr - 1) / kThr;   // per thread
     static constexpr int kWBuf = S * kTileF * kXRowStride;         // bytes of one W ring buffer
-    static constexpr int kXBuf = S * 32 * NB * kXRowStride;        // bytes of one X ring buffer
+    // LDS bytes of one row's sub-step of X: 128, or the three bf16 parts of 32
+    // fp32 values, padded so that the MFMA-layout reads meet no bank conflict
+    static constexpr bool kSplit = DT == DT_F32;
+    static constexpr int kXStride = kSplit ? kXSplitStride : kXRowStride;
+    static constexpr int kXBuf = S * 32 * NB * kXStride;           // bytes of one X ring buffer
     static constexpr int kRingBytes = 2 * kWBuf + 2 * kXBuf;
     static_assert(kXTotal % kThr == 0 || kXChunks == 1, "X chunk split");
     static_assert(kTileF * kRowChunks % kThr == 0, "W chunk split");
@@ -458,9 +493,9 @@ struct TileStream {
         rot = (w_row_bytes & 4095) == 0 ? (int)(((unsigned)x * 7u) % (unsigned)nds) : 0;
     }
 
-    __device__ __forceinline__ int col(int s) const   // column step of step s (s >= nds: any valid one)
+    __device__ __forceinline__ int col(int s) const   // column step of step s < nds
     {
-        const int c = (s < nds ? s : nds - 1) + rot;
+        const int c = s + rot;
         return c >= nds ? c - nds : c;
     }
 
@@ -488,9 +523,10 @@ struct TileStream {
     // apart and share their place in the row.
     __device__ __forceinline__ void issue(u32x4 (&xr)[kXChunks], u32x4 (&wr)[kWChunks])
     {
-        const int s = col(lt < ntiles ? ls : nds);
+        const bool real = lt < ntiles && ls < nds;   // else a padding step: zeros
+        const int s = col(real ? ls : 0);
         const int so = __builtin_amdgcn_readfirstlane(s * (S * kStepBytes));
-        const int to = (tail != 0 && s == nds - 1) ? toff : 0;
+        const int to = !real ? kOut : (tail != 0 && s == nds - 1) ? toff : 0;
 #pragma unroll
         for (int p = 0; p < kXChunks; ++p)
             xr[p] = __builtin_amdgcn_raw_buffer_load_b128(xres, xoff + to, so + p * (kThr / kRowChunks) * (int)w_row_bytes, 0);
@@ -505,29 +541,60 @@ struct TileStream {
         }
     }
 
-    // LDS offset of a thread's chunk p in a ring buffer of `rows` rows per
+    // LDS row of a thread's chunk p in a ring buffer of `rows` rows per
     // 128-byte sub-step
-    __device__ __forceinline__ int ring_off(int p, int rows) const
+    __device__ __forceinline__ int ring_row(int p, int rows) const
     {
         const int c = tid + kThr * p;
-        return (((c % kRowChunks) >> 3) * rows + c / kRowChunks) * kXRowStride + (c & 7) * 16;
+        return ((c % kRowChunks) >> 3) * rows + c / kRowChunks;
     }
 
     __device__ __forceinline__ void store(const u32x4 (&xr)[kXChunks], const u32x4 (&wr)[kWChunks], unsigned char* xs,
                                           unsigned char* wsb) const
     {
 #pragma unroll
-        for (int p = 0; p < kWChunks; ++p) *(u32x4*)(wsb + ring_off(p, kTileF)) = wr[p];
+        for (int p = 0; p < kWChunks; ++p)
+            *(u32x4*)(wsb + ring_row(p, kTileF) * kXRowStride + (tid & 7) * 16) = wr[p];
 #pragma unroll
-        for (int p = 0; p < kXChunks; ++p)
-            if (kXTotal % kThr == 0 || tid < kXTotal) *(u32x4*)(xs + ring_off(p, 32 * NB)) = xr[p];
+        for (int p = 0; p < kXChunks; ++p) store_x(xr[p], p, xs);
+    }
+
+    // A thread's X chunk p to ring buffer xs; fp32 as its three bf16 parts
+    // (X is split here, once for all waves).
+    __device__ __forceinline__ void store_x(const u32x4& v, int p, unsigned char* xs) const
+    {
+        if (kXTotal % kThr != 0 && tid >= kXTotal) return;
+        unsigned char* q = xs + ring_row(p, 32 * NB) * kXStride;
+        if constexpr (kSplit) {
+            uint32_t lo[3], hi[3];
+            split3(__uint_as_float(v[0]), __uint_as_float(v[1]), lo);
+            split3(__uint_as_float(v[2]), __uint_as_float(v[3]), hi);
+#pragma unroll
+            for (int i = 0; i < 3; ++i) *(u32x2*)(q + i * 64 + (tid & 7) * 8) = u32x2{lo[i], hi[i]};
+        } else {
+            *(u32x4*)(q + (tid & 7) * 16) = v;
+        }
+    }
+
+    // compute() of the step in xs / wsb and store() of the loaded chunks to
+    // the other buffers.
+    __device__ __forceinline__ void compute_store(f32x16 (&acc)[NB], const unsigned char* xs, const unsigned char* wsb,
+                                                  const u32x4 (&xr)[kXChunks], const u32x4 (&wr)[kWChunks],
+                                                  unsigned char* xn, unsigned char* wn) const
+    {
+        if constexpr (kSplit) {
+            split_step(acc, xs, wsb, xr, wr, xn, wn);
+        } else {
+            compute(acc, xs, wsb);
+            store(xr, wr, xn, wn);
+        }
     }
 
     __device__ __forceinline__ void compute(f32x16 (&acc)[NB], const unsigned char* xs, const unsigned char* wsb) const
     {
         // wave -> sub-step wave / kLatWaves, latents 32 (wave % kLatWaves) ..:
         // its W rows are ring rows 32 wave ..
-        const unsigned char* xw = xs + (S > 1 ? wave / kLatWaves * (32 * NB) : 0) * kXRowStride;
+        const unsigned char* xw = xs + (S > 1 ? wave / kLatWaves * (32 * NB) : 0) * kXStride;
         u32x4 w[4];
 #pragma unroll
         for (int q = 0; q < 4; ++q) w[q] = *(const u32x4*)(wsb + (wave * 32 + jl) * kXRowStride + h * 64 + q * 16);
@@ -540,7 +607,7 @@ struct TileStream {
             for (int n = 0; n < NP; ++n)
 #pragma unroll
                 for (int q = 0; q < 4; ++q)
-                    bx[n][q] = *(const u32x4*)(xw + (32 * (n0 + n) + jl) * kXRowStride + h * 64 + q * 16);
+                    bx[n][q] = *(const u32x4*)(xw + (32 * (n0 + n) + jl) * kXStride + h * 64 + q * 16);
 #pragma unroll
             for (int q = 0; q < 4; ++q)
 #pragma unroll
@@ -548,14 +615,79 @@ struct TileStream {
         }
     }
 
+    // fp32: compute() of the step in xs / wsb, and store() of the loaded chunks
+    // xr / wr to xn / wn, in one pipeline: 2 NB groups (half g of a lane's
+    // values, row block n) of six MFMAs on the three parts of W and of X, the
+    // smallest products first.  Each group's X parts are read during the group
+    // before, and the splits' VALU work goes between the MFMAs (six fit behind
+    // a 32-cycle MFMA): W's second half during the first NB groups, the next
+    // step's X during the others.  Left to the compiler, the splits ran in
+    // clumps with the MFMAs idle: B = 128, d = 2048, F = 2^18 768 us, 692-729 so
+    // (1044-1072 on the fp32 matrix cores).  What bounds it is the MFMAs at the
+    // power limit's clock: with two of the six products (timing only) 416 us;
+    // splitting by truncation, or one wave of each SIMD storing before its MFMAs
+    // and the other after, changed nothing.
+    __device__ __forceinline__ void split_step(f32x16 (&acc)[NB], const unsigned char* xs, const unsigned char* wsb,
+                                               const u32x4 (&xr)[kXChunks], const u32x4 (&wr)[kWChunks],
+                                               unsigned char* xn, unsigned char* wn) const
+    {
+        const unsigned char* xw = xs + (S > 1 ? wave / kLatWaves * (32 * NB) : 0) * kXStride + jl * kXStride + h * 32;
+        const unsigned char* ww = wsb + (wave * 32 + jl) * kXRowStride + h * 64;
+        u32x4 w[4], wp[2][3], bx[2][3];
+#pragma unroll
+        for (int q = 0; q < 4; ++q) w[q] = *(const u32x4*)(ww + q * 16);
+        auto read_x = [&](int i) {   // parts of group i
+#pragma unroll
+            for (int k = 0; k < 3; ++k)
+                bx[i & 1][k] = *(const u32x4*)(xw + 32 * (i % NB) * kXStride + k * 64 + (i / NB) * 16);
+        };
+        auto split_w = [&](int g, int e) {   // elements 2 e, 2 e + 1 of half g
+            uint32_t pt[3];
+            const u32x4 v = w[2 * g + e / 2];
+            split3(__uint_as_float(v[2 * (e & 1)]), __uint_as_float(v[2 * (e & 1) + 1]), pt);
+#pragma unroll
+            for (int k = 0; k < 3; ++k) wp[g][k][e] = pt[k];
+        };
+        read_x(0);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) split_w(0, e);
+        __builtin_amdgcn_sched_barrier(0);
+        constexpr int pw[6] = {2, 1, 0, 1, 0, 0}, px[6] = {0, 1, 2, 0, 1, 0};
+#pragma unroll
+        for (int i = 0; i < 2 * NB; ++i) {
+            if (i + 1 < 2 * NB) read_x(i + 1);
+            if (i < NB) {
+#pragma unroll
+                for (int e = i * 4 / NB; e < (i + 1) * 4 / NB; ++e) split_w(1, e);
+            } else {
+                const int j = i - NB;
+#pragma unroll
+                for (int p = j * kWChunks / NB; p < (j + 1) * kWChunks / NB; ++p)
+                    *(u32x4*)(wn + ring_row(p, kTileF) * kXRowStride + (tid & 7) * 16) = wr[p];
+#pragma unroll
+                for (int p = j * kXChunks / NB; p < (j + 1) * kXChunks / NB; ++p) store_x(xr[p], p, xn);
+            }
+#pragma unroll
+            for (int k = 0; k < 6; ++k) mfma_quad<DT_BF16>(acc[i % NB], wp[i / NB][pw[k]], bx[i & 1][px[k]]);
+            __builtin_amdgcn_sched_group_barrier(0x100, 3, 0);   // LDS reads
+#pragma unroll
+            for (int k = 0; k < 6; ++k) {
+                __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);   // MFMA
+                __builtin_amdgcn_sched_group_barrier(0x002, 6, 0);   // VALU
+            }
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    }
+
     __device__ __forceinline__ void bias_load(float (&bn)[kTileF / 64], int t) const
     {
-        const int64_t f0 = f_begin + (int64_t)t * kTileF + lane * (kTileF / 64);
+        const int64_t f0 = f_begin + (int64_t)t * kTileF;
+        int64_t n = F - f0;
+        n = n < 0 ? 0 : (n < kTileF ? n : kTileF);   // zeros past the range
+        const __amdgpu_buffer_rsrc_t r = make_rsrc(bias + f0, n * 4);
 #pragma unroll
-        for (int e = 0; e < kTileF / 64; ++e) {
-            const int64_t f = f0 + e;
-            bn[e] = bias[(f < F) ? f : F - 1];
-        }
+        for (int e = 0; e < kTileF / 64; ++e)
+            bn[e] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(r, lane * (kTileF / 64) * 4 + 4 * e, 0, 0));
     }
 
     __device__ __forceinline__ void bias_store(const float (&bn)[kTileF / 64], float* buf) const
@@ -624,6 +756,74 @@ struct TileStream {
         }
     }
 
+    // fp32 (kSplit): whether score s of a latent with bias b may have met an
+    // input that its three bf16 parts do not hold.  An infinite or NaN input,
+    // or one that rounds past bf16's largest value, leaves no finite score
+    // (one that equals an infinite bias, or whose bias is NaN, is right as it is);
+    // inputs so small that their lower parts vanish matter only to a score as
+    // small.  Scores of exactly zero are taken as they are.
+    static constexpr uint32_t kTiny = 0x17800000u, kInf = 0x7F800000u;   // 2^-80, infinity
+    __device__ __forceinline__ static bool suspect(float s, float b)
+    {
+        const uint32_t u = __float_as_uint(s) & 0x7FFFFFFFu, ub = __float_as_uint(b) & 0x7FFFFFFFu;
+        return u != 0u && u - kTiny >= kInf - kTiny && !(u >= kInf && (ub > kInf || s == b));
+    }
+
+    // fp32: scores of tile t that are suspect are recomputed, with all others
+    // of the wave, by the fp32 MFMA from operands read straight from memory:
+    // slow, and reached only by inputs that are not finite, near the largest
+    // float or tiny.
+    __device__ __forceinline__ void fix_up(f32x16 (&acc)[NB], int t, const float* bias_buf) const
+    {
+        if constexpr (kSplit) {
+            if (S > 1 && wave >= kLatWaves) return;
+            uint32_t far = 0;   // a first look that also takes zeros
+#pragma unroll
+            for (int n = 0; n < NB; ++n)
+#pragma unroll
+                for (int r = 0; r < 16; ++r) {
+                    const uint32_t u = (__float_as_uint(acc[n][r]) & 0x7FFFFFFFu) - kTiny;
+                    far = u > far ? u : far;
+                }
+            if (__ballot(far >= kInf - kTiny) == 0) return;
+            float bv[16];
+            bias_read(bv, bias_buf);
+            bool bad = false;
+#pragma unroll
+            for (int n = 0; n < NB; ++n)
+#pragma unroll
+                for (int r = 0; r < 16; ++r) bad |= suspect(acc[n][r], bv[r]);
+            if (__ballot(bad) == 0) return;
+#pragma unroll
+            for (int n = 0; n < NB; ++n)
+#pragma unroll
+                for (int r = 0; r < 16; ++r) acc[n][r] = bv[r];
+            const int64_t f0 = f_begin + (int64_t)t * kTileF;
+            const int64_t nr = F - f0 < kTileF ? F - f0 : kTileF;
+            const __amdgpu_buffer_rsrc_t wr = make_rsrc(W + f0 * w_row_bytes, nr * w_row_bytes);
+            const int nq = (int)(w_row_bytes / 16);   // 16-byte chunks of a row
+            // (the empty asm keeps the row offsets from being formed ahead of the
+            // tile loop and held in registers through it)
+            int jr = jl;
+            asm volatile("" : "+v"(jr));
+#pragma unroll 1
+            for (int c0 = 0; c0 < nq; c0 += 8) {
+#pragma unroll 1
+                for (int q = 0; q < 4; ++q) {
+                    const int c = c0 + 4 * h + q;
+                    const int off = c < nq ? c * 16 : kOut;
+                    const u32x4 w = __builtin_amdgcn_raw_buffer_load_b128(wr, off + (wave * 32 + jr) * (int)w_row_bytes, 0, 0);
+#pragma unroll
+                    for (int n = 0; n < NB; ++n) {
+                        const u32x4 x =
+                            __builtin_amdgcn_raw_buffer_load_b128(xres, off + (32 * n + jr) * (int)w_row_bytes, 0, 0);
+                        mfma_quad<DT_F32>(acc[n], w, x);
+                    }
+                }
+            }
+        }
+    }
+
     template <bool kBiasInit, class Epi>
     __device__ __forceinline__ void run(f32x16 (&acc)[NB], unsigned char* ring, float* bias_lds, Epi epi)
     {
@@ -653,17 +853,16 @@ struct TileStream {
             for (int s = 0; s < nds2; s += 2) {
                 float bn[kTileF / 64];
                 if (wave == 0) bias_load(bn, t + 1);   // past the last tile: clamped, unused
-                if (s < nds) compute(acc, xs0, ws0);
-                store(x1, w1, xs1, ws1);
+                compute_store(acc, xs0, ws0, x1, w1, xs1, ws1);
                 issue(x1, w1);
                 __syncthreads();
-                if (s + 1 < nds) compute(acc, xs1, ws1);
-                store(x0, w0, xs0, ws0);
+                compute_store(acc, xs1, ws1, x0, w0, xs0, ws0);
                 issue(x0, w0);
                 if (wave == 0) bias_store(bn, bnext);
                 __syncthreads();
             }
             reduce(acc, ws1);
+            if (kBiasInit) fix_up(acc, t, bias_lds + (t & 1) * kTileF);
             float bv[16];
             if (!kBiasInit) bias_read(bv, bias_lds + (t & 1) * kTileF);
             epi(t, acc, bv);

@@ -267,12 +267,13 @@ __device__ __forceinline__ void group_tiles(const GroupArgs& a)
     static_assert(TS::kTileF == kGroupTile && kGroupTile == 2 * kApproxGroup, "one tile is two groups");
     extern __shared__ __align__(16) unsigned char smem[];
     float* bias_lds = (float*)(smem + TS::kRingBytes);             // [2][kGroupTile]
-    uint32_t* ordv = (uint32_t*)(bias_lds + 2 * kGroupTile);       // [32 rows][kOrdStride]
-    uint64_t* hbuf = (uint64_t*)(ordv + 32 * kOrdStride);          // [32*NB rows][kHeadSlots] head keys
+    uint64_t* hbuf = (uint64_t*)(bias_lds + 2 * kGroupTile);       // [32*NB rows][kHeadSlots] head keys
+    // [32 rows][kOrdStride] score words, in W ring buffer 1 (idle during the epilogue)
+    uint32_t* ordv = (uint32_t*)(smem + TS::kWBuf);
+    static_assert(32 * kOrdStride * sizeof(uint32_t) <= (size_t)TS::kWBuf, "the words fit the ring buffer");
 
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int h = lane >> 5, jl = lane & 31;
-    const int l = lane & 15, sq = lane >> 4;
     const int64_t b0 = (int64_t)blockIdx.y * (32 * NB);
     const int64_t B = a.B, F = a.F, G = a.num_groups;
     const int64_t num_tiles = (G + 1) / 2;
@@ -303,6 +304,9 @@ __device__ __forceinline__ void group_tiles(const GroupArgs& a)
         const int64_t f0 = tile * kGroupTile;
         // accumulator register r of this lane: row 32n + jl, latent lt0 + 8*(r/4) + r%4
         const int lt0 = wave * 32 + h * 4;
+        int te = tid;   // (hidden, so that nothing derived from it is held in registers through the d-steps)
+        asm volatile("" : "+v"(te));
+        const int l = te & 15, sq = (te >> 4) & 3;
 #pragma unroll
         for (int n = 0; n < NB; ++n) {
             if (n > 0) __syncthreads();   // the previous block's keys are read
@@ -320,7 +324,7 @@ __device__ __forceinline__ void group_tiles(const GroupArgs& a)
             // 64 (row, group) segments per block, 4 per wave and round
 #pragma unroll
             for (int rd = 0; rd < 2; ++rd) {
-                const int seg = wave * 8 + rd * 4 + sq;
+                const int seg = (te >> 6) * 8 + rd * 4 + sq;
                 const int rl = seg >> 1, g = seg & 1;
                 sort_segment<C>(a, ordv, hbuf + 32 * n * kHeadSlots, rl, g, l, b0 + 32 * n, tile);
             }
@@ -340,6 +344,7 @@ __device__ __forceinline__ void group_tiles(const GroupArgs& a)
                 if (row < B && grp >= g0 && grp < g1) a.heads[row * G + grp] = hbuf[i];
             }
         }
+        __syncthreads();   // the words are read: the ring buffer's next writer may come
     });
 }
 
@@ -347,7 +352,7 @@ __device__ __forceinline__ void group_tiles(const GroupArgs& a)
 template <class Kern, int DT, int NB, int C>
 static hipError_t launch_group_c(const GroupArgs& a, dim3 grid, hipStream_t st)
 {
-    const size_t lds = group_lds_bytes(NB);
+    const size_t lds = group_lds_bytes(DT, NB);
     auto kern = Kern::template kernel<DT, NB, C>();
     hipError_t e = ensure_lds((const void*)kern, lds);
     if (e != hipSuccess) return e;

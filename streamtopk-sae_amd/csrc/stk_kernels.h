@@ -212,6 +212,10 @@ struct ThrArgs {
 constexpr int kLargeRows = 256;
 constexpr int kLargeThreads = 256;
 constexpr int64_t kLargeMinB = 512;   // batches from this size use mainl_kernel
+// fp32: main_kernel multiplies on the bf16 matrix cores (split3), mainl_kernel
+// on the fp32 ones, at 2.7 times the cycles; past 2048 rows main_kernel's grid
+// has fewer than kXchMinWg workgroups per row block.
+constexpr int64_t kLargeMinBF32 = 2049;
 constexpr int kLXchPerWg = 4;         // exchanged maxima per row and mainl_kernel workgroup
 
 struct MainLArgs {
@@ -325,10 +329,10 @@ inline bool nontemporal_w(const void* W, int64_t row_bytes, int64_t row_blocks)
     return row_blocks == 1 && (((uintptr_t)W | (uintptr_t)row_bytes) & (kStepBytes - 1)) == 0;
 }
 
-size_t main_lds_bytes(int NB, int S, int cap, int lq);
-int main_lds_queue(int NB, int S, int k);
+size_t main_lds_bytes(int dt, int NB, int S, int cap, int lq);
+int main_lds_queue(int dt, int NB, int S, int k);
 size_t mainl_lds_bytes(int cap);
-size_t group_lds_bytes(int NB);
+size_t group_lds_bytes(int dt, int NB);
 
 hipError_t launch_main(int dt, int NB, int S, const MainArgs& a, dim3 grid, hipStream_t st);
 hipError_t launch_mainl(int dt, const MainLArgs& a, int grid, hipStream_t st);

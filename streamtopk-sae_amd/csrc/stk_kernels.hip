@@ -168,12 +168,14 @@ __device__ __forceinline__ void xch_thresholds(const MainArgs& a, const f32x16 (
 {
     constexpr int BT = 32 * NB;
     const int xper = a.xper, nw = (int)gridDim.x * xper;   // maxima per workgroup and row, per row
+    // the thread's index and the row block pass through empty asms so that no
+    // address derived from them is hoisted out of the tile loop (kept live, it
+    // would spill)
+    asm volatile("" : "+v"(tid));
     const int lane = tid & 63, wave = tid >> 6, h = lane >> 5, jl = lane & 31;
     const int nwg = (int)gridDim.x, x = (int)blockIdx.x;
     const int nrows = (int)(a.B - b0 < BT ? a.B - b0 : BT);
     const int nown = nwg < nrows ? nwg : nrows;
-    // the row block passes through an empty asm so that no address derived
-    // from it is hoisted out of the tile loop (kept live, it would spill)
     int64_t yb = blockIdx.y;
     asm volatile("" : "+s"(yb));
     uint64_t* xmax = a.xmax + yb * BT * nw;    // [BT][nw]
@@ -386,12 +388,15 @@ __global__ __launch_bounds__(kMainThreads, 2) void main_kernel(MainArgs a)
     // segments (compacting a segment without room), then publishes how many
     // keys each of its segments holds ----
     __syncthreads();
-    flush_rows<R>(cnt, gcnt, thr, lqk, seg, a.list_cap, cscr + wave * cap, lq, cap, k, wave, lane);
+    int ft = tid;   // (hidden, so that the flush's addresses are not held in registers through the tiles)
+    asm volatile("" : "+v"(ft));
+    const int fl = ft & 63, fw = ft >> 6;
+    flush_rows<R>(cnt, gcnt, thr, lqk, seg, a.list_cap, cscr + fw * cap, lq, cap, k, fw, fl);
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-    const int myrow = wave * R + lane;
-    if (lane < R && b0 + myrow < B) a.seg_cnt[(b0 + myrow) * gridDim.x + blockIdx.x] = gcnt[myrow];
+    const int myrow = fw * R + fl;
+    if (fl < R && b0 + myrow < B) a.seg_cnt[(b0 + myrow) * gridDim.x + blockIdx.x] = gcnt[myrow];
 }
 
 // ---------------------------------------------------------------------------
@@ -1027,21 +1032,22 @@ __global__ __launch_bounds__(kProbeThreads) void read_probe_kernel(const u32x4* 
 // ---------------------------------------------------------------------------
 // Host-side launch helpers
 // ---------------------------------------------------------------------------
-size_t main_lds_bytes(int NB, int S, int cap, int lq)
+size_t main_lds_bytes(int dt, int NB, int S, int cap, int lq)
 {
     const size_t BT = 32 * (size_t)NB;
-    const size_t rings = 2 * (size_t)kTileLatents * kXRowStride + 2 * S * BT * kXRowStride;   // TileStream rings
+    const size_t xs = dt == DT_F32 ? kXSplitStride : kXRowStride;
+    const size_t rings = 2 * (size_t)kTileLatents * kXRowStride + 2 * S * BT * xs;   // TileStream rings
     return rings + BT * 8 + BT * 8 + 2 * (kTileLatents / S) * 4 + BT * (size_t)lq * 8 + (size_t)kMainWaves * cap * 8 +
            2 * kMainWaves * sizeof(uint32_t);
 }
 
 // LDS queue keys per row: the most (even, at most 64) whose LDS use, with
 // global segments of cap = k + lq keys, fits 159 KiB of the workgroup's 160.
-int main_lds_queue(int NB, int S, int k)
+int main_lds_queue(int dt, int NB, int S, int k)
 {
     for (int lq = 64; lq >= 2; lq -= 2) {
         const int cap = (k + lq + 1) & ~1;
-        if (main_lds_bytes(NB, S, cap, lq) <= 159 * 1024) return lq;
+        if (main_lds_bytes(dt, NB, S, cap, lq) <= 159 * 1024) return lq;
     }
     return 0;
 }
@@ -1049,7 +1055,7 @@ int main_lds_queue(int NB, int S, int k)
 template <int DT, int NB, int S, bool NT>
 static hipError_t launch_main_t(const MainArgs& a, dim3 grid, hipStream_t st)
 {
-    const size_t lds = main_lds_bytes(NB, S, a.cap, a.lq);
+    const size_t lds = main_lds_bytes(DT, NB, S, a.cap, a.lq);
     auto kern = main_kernel<DT, NB, S, NT>;
     hipError_t e = ensure_lds((const void*)kern, lds);
     if (e != hipSuccess) return e;
