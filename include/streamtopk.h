@@ -122,6 +122,13 @@ int stk_topk_merge_workspace_bytes(int64_t B, int64_t k, int64_t nparts, size_t*
 int stk_topk_merge(const float* Vp, const int32_t* Ip, int64_t nparts, int64_t B, int64_t k,
                    float* V, int32_t* I, void* workspace, size_t workspace_bytes, void* stream);
 
+/* stk_topk_merge over parts that lie apart: Vp[p] / Ip[p] are part p's (B, k)
+ * device arrays (the pointer arrays themselves are host memory, read during
+ * the call).  At most 16 parts with nparts * k <= 4096; no workspace.  The
+ * same result as stk_topk_merge of the stacked parts. */
+int stk_topk_merge_parts(const float* const* Vp, const int32_t* const* Ip, int64_t nparts, int64_t B,
+                         int64_t k, float* V, int32_t* I, void* stream);
+
 /* Device workspace (bytes) for stk_approx_forward.  `with_candidates` is
  * non-zero when the caller passes a candidate buffer (then the workspace holds
  * 256 bytes, then each group's first candidate as an 8-byte key:

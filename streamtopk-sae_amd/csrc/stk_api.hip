@@ -821,6 +821,49 @@ int stk_topk_merge_workspace_bytes(int64_t B, int64_t k, int64_t nparts, size_t*
     return 0;
 }
 
+// Whether the parts are merged where they lie (merge_parts_kernel).
+static bool merge_in_place(int64_t k, int64_t nparts) { return nparts <= kMaxParts && nparts * k <= kSelCap; }
+
+static int run_merge_parts(const float* const* Vp, const int32_t* const* Ip, int64_t nparts, int64_t B, int64_t k,
+                           float* V, int32_t* I, hipStream_t st)
+{
+    PartsArgs a;
+    std::memset(&a, 0, sizeof a);
+    for (int64_t p = 0; p < nparts; ++p) {
+        a.V[p] = Vp[p];
+        a.I[p] = Ip[p];
+    }
+    a.nparts = (int)nparts;
+    a.k = (int)k;
+    a.Vo = V;
+    a.Io = I;
+    const int pg = prof_begin("merge_kernel", st);
+    const hipError_t e = launch_merge_parts(a, B, st);
+    prof_end(pg, st);
+    if (e != hipSuccess) return hip_fail(e, "merge_parts_kernel launch");
+    return 0;
+}
+
+int stk_topk_merge_parts(const float* const* Vp, const int32_t* const* Ip, int64_t nparts, int64_t B, int64_t k,
+                         float* V, int32_t* I, void* stream)
+{
+    clear_error();
+    int rc = validate_merge(B, k, nparts);
+    if (rc) return rc;
+    if (!merge_in_place(k, nparts))
+        return set_error(STK_E_INVALID, "at most %d parts and %d entries per row can be merged in place", kMaxParts,
+                         kSelCap);
+    if (B == 0) return 0;
+    if (!Vp || !Ip || !V || !I) return set_error(STK_E_INVALID, "null tensor pointer");
+    uintptr_t all = (uintptr_t)V | (uintptr_t)I;
+    for (int64_t p = 0; p < nparts; ++p) {
+        if (!Vp[p] || !Ip[p]) return set_error(STK_E_INVALID, "null tensor pointer");
+        all |= (uintptr_t)Vp[p] | (uintptr_t)Ip[p];
+    }
+    if (all & 3) return set_error(STK_E_INVALID, "values and indices must be 4-byte aligned");
+    return run_merge_parts(Vp, Ip, nparts, B, k, V, I, (hipStream_t)stream);
+}
+
 int stk_topk_merge(const float* Vp, const int32_t* Ip, int64_t nparts, int64_t B, int64_t k,
                    float* V, int32_t* I, void* workspace, size_t workspace_bytes, void* stream)
 {
@@ -838,6 +881,15 @@ int stk_topk_merge(const float* Vp, const int32_t* Ip, int64_t nparts, int64_t B
     if ((uintptr_t)workspace & 255) return set_error(STK_E_INVALID, "workspace must be 256-byte aligned");
     unsigned char* ws = (unsigned char*)workspace;
     const hipStream_t st = (hipStream_t)stream;
+    if (merge_in_place(k, nparts)) {
+        const float* Vq[kMaxParts];
+        const int32_t* Iq[kMaxParts];
+        for (int64_t p = 0; p < nparts; ++p) {
+            Vq[p] = Vp + p * B * k;
+            Iq[p] = Ip + p * B * k;
+        }
+        return run_merge_parts(Vq, Iq, nparts, B, k, V, I, st);
+    }
     PackArgs pa;
     pa.V = Vp; pa.I = Ip; pa.B = B; pa.k = (int)k; pa.nparts = (int)nparts;
     pa.list_keys = (uint64_t*)(ws + kCtlBytes);

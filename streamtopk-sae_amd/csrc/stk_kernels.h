@@ -295,6 +295,18 @@ struct PackArgs {                // partial top-k results -> dense candidate lis
     int64_t list_cap;
 };
 
+// Partial results merged by merge_parts_kernel: at most this many, of at most
+// kSelCap entries per row together (more go through pack_kernel).
+constexpr int kMaxParts = 16;
+
+struct PartsArgs {
+    const float* V[kMaxParts];   // [B][k] each
+    const int32_t* I[kMaxParts]; // [B][k] latent indices
+    int nparts, k;               // k a power of two
+    float* Vo;                   // [B][k]
+    int32_t* Io;
+};
+
 struct GroupArgs {               // approximate variant, per-group top-c candidates
     const void* X;
     const void* W;
@@ -341,6 +353,7 @@ hipError_t launch_sample(int dt, int NB, const SampleArgs& a, dim3 grid, hipStre
 hipError_t launch_thr(const ThrArgs& a, int64_t rows, hipStream_t st);
 hipError_t launch_merge(const MergeArgs& a, int64_t rows, hipStream_t st);
 hipError_t launch_pack(const PackArgs& a, int64_t rows, hipStream_t st);
+hipError_t launch_merge_parts(const PartsArgs& a, int64_t rows, hipStream_t st);
 hipError_t launch_group(int dt, int NB, const GroupArgs& a, dim3 grid, hipStream_t st);
 hipError_t launch_group_cached(int dt, int NB, const GroupArgs& a, dim3 grid, hipStream_t st);
 hipError_t launch_cand(const CandArgs& a, int64_t rows, hipStream_t st);

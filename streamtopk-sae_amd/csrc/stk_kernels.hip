@@ -954,6 +954,93 @@ __global__ __launch_bounds__(kThreads) void pack_kernel(PackArgs a)
 }
 
 // ---------------------------------------------------------------------------
+// merge_parts_kernel: top-k of up to kMaxParts partial results read where they
+// are, kPer entries per thread, one workgroup per row: one launch instead of
+// stacking the parts, packing them as keys and merging the lists.  Parts are
+// usually in descending order (what the encoder returns): then the smallest
+// of the parts' entries ceil(k / nparts) is reached by k entries, and the
+// few entries that reach it (~1.4 k) are ranked by counting; other parts go
+// through the merges' pass.  A latency chain: loads, votes, selection.
+// 8 parts, B = 1024, k = 128, per call: stacked, packed and merged 34 us; in
+// place through the merges' pass (1024 entries: a radix selection) 18 us.
+// ---------------------------------------------------------------------------
+template <int kPer>
+__global__ __launch_bounds__(kThreads) void merge_parts_kernel(PartsArgs a)
+{
+    __shared__ SelShared S;
+    __shared__ const float* pv[kMaxParts];
+    __shared__ const int32_t* pi[kMaxParts];
+    __shared__ uint64_t tk[kMaxParts];
+    const int tid = threadIdx.x, lane = tid & 63, k = a.k;
+    const int64_t row = blockIdx.x;
+    // the pointers by place in LDS (a lane cannot index the kernel's arguments)
+#pragma unroll
+    for (int p = 0; p < kMaxParts; ++p)
+        if (tid == p) {
+            pv[p] = a.V[p];
+            pi[p] = a.I[p];
+        }
+    if (tid == 0) S.cnt = 0;
+    __syncthreads();
+    const int n = a.nparts * k, sh = __builtin_ctz(k);
+    // entry i is entry i % k of part i / k; lane 0 also loads entry i - 1
+    // (its neighbour lies in another wave)
+    float val[kPer], pval[kPer];
+    int32_t idx[kPer], pidx[kPer];
+#pragma unroll
+    for (int u = 0; u < kPer; ++u) {
+        const int i = tid + u * kThreads;
+        if (i < n) {
+            const float* vp = pv[i >> sh];
+            const int32_t* ip = pi[i >> sh];
+            const int64_t src = row * k + (i & (k - 1));
+            val[u] = vp[src];
+            idx[u] = ip[src];
+            if (lane == 0 && (i & (k - 1)) != 0) {
+                pval[u] = vp[src - 1];
+                pidx[u] = ip[src - 1];
+            }
+        }
+    }
+    const int rb = (k + a.nparts - 1) / a.nparts - 1;
+    uint64_t v[kPer];
+    bool rising = false;
+#pragma unroll
+    for (int u = 0; u < kPer; ++u) {
+        const int i = tid + u * kThreads;
+        const bool in = i < n;
+        v[u] = in ? make_key(val[u], idx[u]) : 0ull;
+        const uint32_t lo = __shfl_up((uint32_t)v[u], 1), hi = __shfl_up((uint32_t)(v[u] >> 32), 1);
+        uint64_t pk = ((uint64_t)hi << 32) | lo;
+        if (in && (i & (k - 1)) != 0) {
+            if (lane == 0) pk = make_key(pval[u], pidx[u]);
+            rising |= pk < v[u];
+        }
+        if (in && (i & (k - 1)) == rb) tk[i >> sh] = v[u];
+    }
+    uint32_t vpar = 0;
+    if (block_any<kThreads / 64>(rising, S.vote, vpar, tid >> 6, lane)) {
+        uint64_t run = 0;
+        merge_pass(S, v, k, tid, run, vpar);
+    } else {
+        uint64_t T = ~0ull;
+        for (int p = 0; p < a.nparts; ++p) T = tk[p] < T ? tk[p] : T;
+        int c = 0;
+#pragma unroll
+        for (int u = 0; u < kPer; ++u) c += (v[u] != 0 && v[u] >= T) ? 1 : 0;
+        int pos = wave_reserve(&S.cnt, c);   // n <= kSelCap entries in all
+#pragma unroll
+        for (int u = 0; u < kPer; ++u)
+            if (v[u] != 0 && v[u] >= T) S.buf[pos++] = v[u];
+    }
+    // the parts may repeat a latent: equal keys take consecutive ranks
+    emit_topk<true>(S, k, tid, [&](int r, uint64_t kk) {
+        a.Vo[row * k + r] = key_value(kk);
+        a.Io[row * k + r] = key_index(kk);
+    });
+}
+
+// ---------------------------------------------------------------------------
 // fill_zero_kernel: n16 16-byte words at p set to zero, grid-stride.
 // ---------------------------------------------------------------------------
 __global__ __launch_bounds__(kThreads) void fill_zero_kernel(u32x4* p, int64_t n16)
@@ -1138,6 +1225,20 @@ hipError_t launch_fill_zero(void* p, size_t bytes, hipStream_t st)
 hipError_t launch_pack(const PackArgs& a, int64_t rows, hipStream_t st)
 {
     launch(pack_kernel, dim3((unsigned)rows), dim3(kThreads), 0, st, a);
+    return hipGetLastError();
+}
+
+hipError_t launch_merge_parts(const PartsArgs& a, int64_t rows, hipStream_t st)
+{
+    const int n = a.nparts * a.k;
+    if (n <= kThreads)
+        launch(merge_parts_kernel<1>, dim3((unsigned)rows), dim3(kThreads), 0, st, a);
+    else if (n <= 4 * kThreads)
+        launch(merge_parts_kernel<4>, dim3((unsigned)rows), dim3(kThreads), 0, st, a);
+    else if (n <= kSelCap)
+        launch(merge_parts_kernel<kSelCap / kThreads>, dim3((unsigned)rows), dim3(kThreads), 0, st, a);
+    else
+        return hipErrorInvalidValue;
     return hipGetLastError();
 }
 

@@ -14,6 +14,8 @@ LIB_PATH = os.path.join(_HERE, "libstreamtopk_hip.so")
 STK_DTYPE_F32 = 0
 STK_DTYPE_F16 = 1
 STK_DTYPE_BF16 = 2
+STK_E_INVALID = 1
+STK_E_WORKSPACE = 3
 ABI_VERSION = 1
 
 # Every symbol include/streamtopk.h declares, with its ctypes signature.
@@ -32,6 +34,7 @@ SIGNATURES = {
     "stk_exact_forward_noalloc": (_int, [_vp, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _i64, _int, _vp]),
     "stk_topk_merge_workspace_bytes": (_int, [_i64, _i64, _i64, _szp]),
     "stk_topk_merge": (_int, [_vp, _vp, _i64, _i64, _i64, _vp, _vp, _vp, ctypes.c_size_t, _vp]),
+    "stk_topk_merge_parts": (_int, [_vp, _vp, _i64, _i64, _i64, _vp, _vp, _vp]),
     "stk_approx_workspace_bytes": (_int, [_i64, _i64, _i64, _i64, _i64, _int, _int, _szp]),
     "stk_approx_forward": (_int, [_vp, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _i64, _i64, _int,
                                   _vp, _vp, _vp, ctypes.c_size_t, _vp]),

@@ -21,6 +21,7 @@ library requires before a workspace's first use; calls leave it valid for the
 next, and a call that fails drops it.  ``clear_workspace_cache()`` releases
 them.
 """
+import contextlib
 import ctypes
 import threading
 
@@ -36,7 +37,15 @@ _DTYPES = {
 
 
 def _ptr(t):
-    return ctypes.c_void_p(t.data_ptr()) if t is not None else None
+    return t.data_ptr() if t is not None else None
+
+
+def _on_device(device):
+    """Context in which `device` is the current one (entering and leaving the
+    device it already is would cost a small call more than its checks do)."""
+    if torch._C._cuda_getDevice() == device.index:
+        return contextlib.nullcontext()
+    return torch.cuda.device(device)
 
 
 _WS = {}                      # (device index, stream handle) -> uint8 device tensor
@@ -55,6 +64,24 @@ def _workspace(device, stream, nbytes):
             ws = torch.zeros(max(nbytes, 1), dtype=torch.uint8, device=device)
             _WS[key] = ws
         return ws
+
+
+def _run(device, stream, size_of, call):
+    """call(workspace address, its bytes) with the stream's workspace.  The
+    library checks the size before any device work, so the size a call needs
+    (size_of, which plans it) is asked for only when there is no workspace yet
+    or it is too small."""
+    ws = _WS.get((device.index, stream))
+    rc = call(ws.data_ptr(), ws.numel()) if ws is not None else _lib.STK_E_WORKSPACE
+    if rc == _lib.STK_E_WORKSPACE:
+        nbytes = ctypes.c_size_t(0)
+        _lib.check(size_of(ctypes.byref(nbytes)))
+        ws = _workspace(device, stream, nbytes.value)
+        rc = call(ws.data_ptr(), ws.numel())
+    if rc == _lib.STK_E_INVALID:
+        _lib.check(rc)   # rejected before any device work: the workspace is as it was
+    if rc:
+        _check_drop(rc, device, stream)
 
 
 def _check_drop(rc, device, stream):
@@ -182,31 +209,56 @@ def _device_inputs(X, W_enc, b_enc):
     return _aligned(X), _aligned(W_enc), b_enc
 
 
+def _operands(X, W_enc, b_enc):
+    """(X, W_enc, b_enc, their addresses, B, d, F, dtype code, device) after the
+    checks, and the padding and alignment, of _device_inputs.  Inputs that need
+    neither pass one test; the others take the checks one by one."""
+    xs, ws, device, dtype = X.shape, W_enc.shape, X.device, X.dtype
+    code = _DTYPES.get(dtype)
+    x, w = X.data_ptr(), W_enc.data_ptr()
+    if not (X.is_cuda and code is not None and W_enc.dtype is dtype and b_enc.dtype is torch.float32
+            and W_enc.device == device and b_enc.device == device
+            and len(xs) == 2 and len(ws) == 2 and b_enc.dim() == 1 and ws[1] == xs[1] and b_enc.shape[0] == ws[0]
+            and X.is_contiguous() and W_enc.is_contiguous() and b_enc.is_contiguous()
+            and (x | w) % 16 == 0 and xs[1] % (4 if dtype is torch.float32 else 8) == 0):
+        X, W_enc, b_enc = _device_inputs(X, W_enc, b_enc)
+        xs, ws, x, w = X.shape, W_enc.shape, X.data_ptr(), W_enc.data_ptr()
+    return X, W_enc, b_enc, x, w, b_enc.data_ptr(), xs[0], xs[1], ws[0], code, device
+
+
+def _refused_k(k):
+    """Whether k cannot be the size of an output that is allocated before the
+    library has looked at k."""
+    return type(k) is not int or not 0 <= k <= 128
+
+
 def exact_forward(X, W_enc, b_enc, k, f_offset=0):
     """The native exact forward (streamtopk_exact.cu:788-833): contiguous device
     tensors, fp32 b_enc; returns (V fp32 (B,k), I int32 (B,k)).  A non-zero
     f_offset marks W_enc / b_enc as latents f_offset .. f_offset+F-1 of a
     larger dictionary (one shard): the indices are global."""
     lib = _lib.load()
-    X, W_enc, b_enc = _device_inputs(X, W_enc, b_enc)
-    B, d = X.shape
-    F = W_enc.shape[0]
-    dt = _DTYPES[X.dtype]
-    with torch.cuda.device(X.device):
-        nbytes = ctypes.c_size_t(0)
-        _lib.check(lib.stk_exact_workspace_bytes(B, d, F, k, dt, ctypes.byref(nbytes)))
-        V = torch.empty((B, k), dtype=torch.float32, device=X.device)
-        I = torch.empty((B, k), dtype=torch.int32, device=X.device)
-        stream = torch.cuda.current_stream(X.device).cuda_stream
-        ws = _workspace(X.device, stream, nbytes.value)
+    X, W_enc, b_enc, x, w, b, B, d, F, dt, device = _operands(X, W_enc, b_enc)
+
+    def size_of(out):
+        return lib.stk_exact_workspace_bytes(B, d, F, k, dt, out)
+
+    with _on_device(device):
+        if _refused_k(k):
+            _lib.check(size_of(ctypes.byref(ctypes.c_size_t(0))))
+        V = torch.empty((B, k), dtype=torch.float32, device=device)
+        I = torch.empty((B, k), dtype=torch.int32, device=device)
+        v, i = V.data_ptr(), I.data_ptr()
+        stream = torch._C._cuda_getCurrentRawStream(device.index)
         if f_offset:
-            rc = lib.stk_exact_forward_shard(_ptr(X), _ptr(W_enc), _ptr(b_enc), _ptr(V), _ptr(I),
-                                             B, d, F, k, dt, int(f_offset), _ptr(ws), ws.numel(),
-                                             ctypes.c_void_p(stream))
+            off = int(f_offset)
+
+            def call(ws, n):
+                return lib.stk_exact_forward_shard(x, w, b, v, i, B, d, F, k, dt, off, ws, n, stream)
         else:
-            rc = lib.stk_exact_forward(_ptr(X), _ptr(W_enc), _ptr(b_enc), _ptr(V), _ptr(I),
-                                       B, d, F, k, dt, _ptr(ws), ws.numel(), ctypes.c_void_p(stream))
-        _check_drop(rc, X.device, stream)
+            def call(ws, n):
+                return lib.stk_exact_forward(x, w, b, v, i, B, d, F, k, dt, ws, n, stream)
+        _run(device, stream, size_of, call)
     return V, I
 
 
@@ -227,6 +279,35 @@ def topk_sae_cuda_exact(X, W_enc, b_enc, k, *, f_offset=0):
     return exact_forward(X.contiguous(), W_enc.contiguous(), b_enc.contiguous(), k, f_offset=f_offset)
 
 
+def _parts_in_place(values, indices, k):
+    """The parts' addresses (two pointer arrays), B and the device, if they are
+    sequences of contiguous (B, k) device tensors few enough to be merged where
+    they lie; None if not (stacked tensors, other counts, and whatever has to
+    be refused)."""
+    if not (isinstance(values, (list, tuple)) and isinstance(indices, (list, tuple))):
+        return None
+    n = len(values)
+    if not 1 <= n <= 16 or len(indices) != n or k not in (1, 2, 4, 8, 16, 32, 64, 128) or n * k > 4096:
+        return None
+    first = values[0]
+    if not torch.is_tensor(first) or not first.is_cuda or first.dim() != 2:
+        return None
+    shape, place = first.shape, first.get_device()
+    if shape[1] != k:
+        return None
+    vp, ip = [], []
+    for v, i in zip(values, indices):
+        if not (isinstance(v, torch.Tensor) and isinstance(i, torch.Tensor)
+                and v.dtype is torch.float32 and i.dtype is torch.int32
+                and v.shape == shape and i.shape == shape and v.get_device() == place and i.get_device() == place
+                and v.is_contiguous() and i.is_contiguous()):
+            return None
+        vp.append(v.data_ptr())
+        ip.append(i.data_ptr())
+    arr = ctypes.c_void_p * n
+    return arr(*vp), arr(*ip), shape[0], first.device
+
+
 def merge_topk_shards(values, indices, k):
     """Top-k of per-shard top-k results (no counterpart in the reference).
 
@@ -237,6 +318,15 @@ def merge_topk_shards(values, indices, k):
     int32), rows sorted by value descending, equal values by lower index.
     """
     lib = _lib.load()
+    parts = _parts_in_place(values, indices, k)
+    if parts is not None:
+        vp, ip, B, device = parts
+        with _on_device(device):
+            V = torch.empty((B, k), dtype=torch.float32, device=device)
+            I = torch.empty((B, k), dtype=torch.int32, device=device)
+            _lib.check(lib.stk_topk_merge_parts(vp, ip, len(vp), B, k, V.data_ptr(), I.data_ptr(),
+                                                torch._C._cuda_getCurrentRawStream(device.index)))
+        return V, I
     Vp = values if torch.is_tensor(values) else torch.stack(list(values))
     Ip = indices if torch.is_tensor(indices) else torch.stack(list(indices))
     if Vp.dim() != 3 or tuple(Ip.shape) != tuple(Vp.shape):
@@ -267,13 +357,14 @@ def approx_forward(X, W_enc, b_enc, k, c, candidate_buffer=None, candidates=Fals
     candidate tensors, shape (B, ceil(F/128), c), are None unless
     `candidates` is set or a `candidate_buffer` is given."""
     lib = _lib.load()
-    X, W_enc, b_enc = _device_inputs(X, W_enc, b_enc)
-    B, d = X.shape
-    F = W_enc.shape[0]
-    dt = _DTYPES[X.dtype]
+    X, W_enc, b_enc, x, w, b, B, d, F, dt, device = _operands(X, W_enc, b_enc)
     nt = (F + 127) // 128
-    with torch.cuda.device(X.device):
-        with_cand = candidate_buffer is not None or candidates
+    with_cand = candidate_buffer is not None or candidates
+
+    def size_of(out):
+        return lib.stk_approx_workspace_bytes(B, d, F, k, c, dt, int(with_cand), out)
+
+    with _on_device(device):
         cand_vals = cand_idxs = None
         copy_back = None
         if with_cand:
@@ -281,7 +372,7 @@ def approx_forward(X, W_enc, b_enc, k, c, candidate_buffer=None, candidates=Fals
                 cb = candidate_buffer
                 if cb.dim() != 3 or tuple(cb.shape) != (B, nt, c):
                     raise RuntimeError("candidate_buffer shape mismatch")
-                if cb.dtype != torch.float32 or cb.device != X.device or not cb.is_contiguous():
+                if cb.dtype != torch.float32 or cb.device != device or not cb.is_contiguous():
                     raise RuntimeError("candidate_buffer must be a contiguous fp32 tensor on X's device")
                 if cb.data_ptr() % 16:
                     # the kernel writes 16-byte vectors: fill an aligned buffer, then copy
@@ -289,19 +380,19 @@ def approx_forward(X, W_enc, b_enc, k, c, candidate_buffer=None, candidates=Fals
                     cb = torch.empty_like(cb)
                 cand_vals = cb
             else:
-                cand_vals = torch.empty((B, nt, c), dtype=torch.float32, device=X.device)
-            cand_idxs = torch.empty((B, nt, c), dtype=torch.int32, device=X.device)
-        nbytes = ctypes.c_size_t(0)
-        _lib.check(lib.stk_approx_workspace_bytes(B, d, F, k, c, dt, int(with_cand),
-                                                  ctypes.byref(nbytes)))
-        V = torch.empty((B, k), dtype=torch.float32, device=X.device)
-        I = torch.empty((B, k), dtype=torch.int32, device=X.device)
-        stream = torch.cuda.current_stream(X.device).cuda_stream
-        ws = _workspace(X.device, stream, nbytes.value)
-        rc = lib.stk_approx_forward(_ptr(X), _ptr(W_enc), _ptr(b_enc), _ptr(V), _ptr(I),
-                                    B, d, F, k, c, dt, _ptr(cand_vals), _ptr(cand_idxs),
-                                    _ptr(ws), ws.numel(), ctypes.c_void_p(stream))
-        _check_drop(rc, X.device, stream)
+                cand_vals = torch.empty((B, nt, c), dtype=torch.float32, device=device)
+            cand_idxs = torch.empty((B, nt, c), dtype=torch.int32, device=device)
+        if _refused_k(k):
+            _lib.check(size_of(ctypes.byref(ctypes.c_size_t(0))))
+        V = torch.empty((B, k), dtype=torch.float32, device=device)
+        I = torch.empty((B, k), dtype=torch.int32, device=device)
+        v, i, cv, ci = V.data_ptr(), I.data_ptr(), _ptr(cand_vals), _ptr(cand_idxs)
+        stream = torch._C._cuda_getCurrentRawStream(device.index)
+
+        def call(ws, n):
+            return lib.stk_approx_forward(x, w, b, v, i, B, d, F, k, c, dt, cv, ci, ws, n, stream)
+
+        _run(device, stream, size_of, call)
         if copy_back is not None:
             copy_back.copy_(cand_vals)
             cand_vals = copy_back
