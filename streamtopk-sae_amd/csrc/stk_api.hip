@@ -207,19 +207,14 @@ static ExactPlan make_exact_plan(int64_t B, int64_t d, int64_t F, int64_t k, int
     p.xper = 1;
     const int64_t nds = cdiv(d, dtype == STK_DTYPE_F32 ? 32 : 64);   // 128-byte sub-steps of d, the last maybe partial
     int64_t wg_latents = 0;      // main_kernel: latents of a workgroup (at most)
-    if (p.large) {
-        // 256-row blocks; W ranges a multiple of 8 so each range's row blocks share an XCD
-        p.NB = kLargeRows / 32;
-        p.cap = (int)(k + 64 < 192 ? k + 64 : 192);
-        if (p.cap & 1) ++p.cap;
-        p.nbc = cdiv(B, kLargeRows);
-        int64_t nr = ncu / p.nbc;
-        if (nr < 1) nr = 1;
-        if (nr >= 8) nr &= ~(int64_t)7;
-        if (nr > kMergeMaxSeg) nr = kMergeMaxSeg;   // merge_kernel's segments per row
-        p.tpw = cdiv(p.num_tiles, nr);
-        p.nwg = (int)nr;
-    } else {
+    // W ranges of mainl_kernel: a multiple of 8 so each range's row blocks share
+    // an XCD, at most merge_kernel's segments per row
+    const int64_t lnbc = cdiv(B, kLargeRows);
+    int64_t lnr = ncu / (lnbc > 0 ? lnbc : 1);
+    if (lnr < 1) lnr = 1;
+    if (lnr >= 8) lnr &= ~(int64_t)7;
+    if (lnr > kMergeMaxSeg) lnr = kMergeMaxSeg;
+    if (!p.large) {
         // Tiles of 256 / S latents, S sub-steps of d per step (split over the
         // waves; TileStream): the same bytes of W per step.  The S with the
         // fewest steps on the busiest workgroup is taken, a tile's epilogue
@@ -263,6 +258,27 @@ static ExactPlan make_exact_plan(int64_t B, int64_t d, int64_t F, int64_t k, int
         // score was a candidate: B = 128, d = 2048, F = 8192, k = 64 took 391
         // us, 33 us so.)
         while (p.xper * 2 <= kMainWaves / p.S && p.nwg * p.xper * 2 <= 256) p.xper *= 2;
+        // Past two of its row blocks, mainl_kernel's two of 256 rows read W
+        // fewer times, but its tiles are larger: the one with the smaller
+        // estimate runs.  A step of main_kernel takes ~1.3 us and of mainl_kernel
+        // ~1.5, its epilogue ~7, its larger exchange and merge ~8 more.  bf16, step, us, main_kernel / mainl_kernel:
+        // B = 300, d = 2048, F = 2^18 635 / 474, F = 2^16 173 / 134; B = 384,
+        // d = 4096, F = 2^15 242 / 140; but B = 300, d = 768, F = 2^14 35 / 46,
+        // F = 33000 (129 tiles on 128 ranges) 56 / 68, d = 192, F = 24379 36 / 38.  (At up to 256 rows its
+        // one row block is no faster at F = 2^16, and its workspace would pass
+        // the static scratch of the no-allocation calls.)
+        if (dtype != STK_DTYPE_F32 && B > kLargeRows)
+            p.large = (double)cdiv(p.num_tiles, lnr) * (1.5 * (double)nds + 7.0) + 8.0 < 1.3 * (double)best;
+    }
+    if (p.large) {
+        p.S = 1;
+        p.xper = 1;
+        p.NB = kLargeRows / 32;
+        p.cap = (int)(k + 64 < 192 ? k + 64 : 192);
+        if (p.cap & 1) ++p.cap;
+        p.nbc = lnbc;
+        p.tpw = cdiv(p.num_tiles, lnr);
+        p.nwg = (int)lnr;
     }
 
     // The thresholds come from the streaming kernel's own first tiles (each

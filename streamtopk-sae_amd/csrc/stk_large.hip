@@ -134,6 +134,7 @@ struct BigStream {
 
     // load cursors (absolute d-steps), uniform
     int ws, xs;
+    int rot;                     // step s reads the columns of step (s + rot) % s_hi
     __amdgpu_buffer_rsrc_t wres, xres, zres;      // wres: this wave's 64-row run of the tile
     // LDS load i of a wave reads rows 8 i + lane / 8 of the wave's 64-row run
     // (W: of the tile; X: of the row block), chunk lane % 8 ^ xswz(row).
@@ -170,6 +171,12 @@ struct BigStream {
         zres = make_rsrc(X, 0);
     }
 
+    __device__ __forceinline__ int col(int s) const   // column step of step s
+    {
+        const int c = s + rot;
+        return c >= s_hi ? c - s_hi : c;
+    }
+
     __device__ __forceinline__ void begin_tile(int t)
     {
         ws = xs = s_lo;
@@ -199,8 +206,9 @@ struct BigStream {
         const int w = __builtin_amdgcn_readfirstlane(ws);
         const bool live = w < s_hi;
         const __amdgpu_buffer_rsrc_t r = live ? wres : zres;
-        const int so = live ? w * kStepBytes : 0;
-        const bool tl = tail != 0 && w == nds - 1;
+        const int c = col(w);
+        const int so = live ? c * kStepBytes : 0;
+        const bool tl = tail != 0 && c == nds - 1;
         const int b[2] = {tl ? vbt[0] : vb[0], tl ? vbt[1] : vb[1]};
 #pragma unroll
         for (int i = 0; i < kLWChunks; ++i) lds_load16(r, wst + (wave * 64 + 8 * i) * kStepBytes, load_off(b, i), so);
@@ -213,8 +221,9 @@ struct BigStream {
         const int x = __builtin_amdgcn_readfirstlane(xs);
         const bool live = x < s_hi;
         const __amdgpu_buffer_rsrc_t r = live ? xres : zres;
-        const int so = live ? x * kStepBytes : 0;
-        const bool tl = tail != 0 && x == nds - 1;
+        const int c = col(x);
+        const int so = live ? c * kStepBytes : 0;
+        const bool tl = tail != 0 && c == nds - 1;
         const int b[2] = {tl ? vbt[0] : vb[0], tl ? vbt[1] : vb[1]};
 #pragma unroll
         for (int i = 0; i < kLXChunks; ++i)
@@ -249,10 +258,11 @@ struct BigStream {
         const int w = __builtin_amdgcn_readfirstlane(ws);   // the next d-step (ws == xs)
         const bool live = w < s_hi;
         const __amdgpu_buffer_rsrc_t wr = live ? wres : zres, xr = live ? xres : zres;
-        const int so = live ? w * kStepBytes : 0;
+        const int c = col(w);
+        const int so = live ? c * kStepBytes : 0;
         // the next d-step is the partial last one (only kernels built for a
         // partial last step look)
-        const bool tl = TAILK && w == nds - 1;
+        const bool tl = TAILK && live && c == nds - 1;
         // the loads' offsets are formed in the step from two registers: opaque
         // here, so that the compiler does not keep all 16 alive across the loop
         int ob[2] = {tl ? vbt[0] : vb[0], tl ? vbt[1] : vb[1]};
@@ -422,6 +432,7 @@ __global__ __launch_bounds__(kLargeThreads, 1) void mainl_kernel(MainLArgs a)
     bs.nds = (int)((a.d + Dt<DT>::DS - 1) / Dt<DT>::DS);
     bs.tail = (int)(a.d % Dt<DT>::DS);
     bs.samp_log2 = a.samp_log2;
+    bs.rot = 0;
     if (SAMPLE) {
         bs.tile_begin = rg;
         bs.ntiles = 1;
@@ -434,6 +445,14 @@ __global__ __launch_bounds__(kLargeThreads, 1) void mainl_kernel(MainLArgs a)
         bs.ntiles = nt > 0 ? (int)nt : 0;
         bs.s_lo = 0;
         bs.s_hi = bs.nds;
+        // Rows that are a multiple of 4 KiB: each XCD (W range rg runs on XCD
+        // rg % 8) starts at another eighth of the columns, so that the
+        // workgroups, which start together, do not meet on few memory channels
+        // (B = 512, d = 2048, F = 65536: 134 -> 125 us; B = 600, d = 4096 370 ->
+        // 353; B = 1024, d = 4096, F = 2^18 unchanged).  Within an XCD they share
+        // the columns, and with them X in L2: another column per workgroup took
+        // the last 7 % longer.
+        if ((bs.row_bytes & 4095) == 0) bs.rot = ((rg & 7) * bs.nds) >> 3;
     }
     bs.nds2 = (bs.s_hi - bs.s_lo + 1) / 2 * 2;
     bs.tid = tid;
