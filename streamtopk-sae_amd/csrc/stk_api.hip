@@ -196,8 +196,10 @@ struct ExactPlan {
     size_t off_thr, off_list, off_lcnt, off_seg, off_xmax, off_xthr, total;
 };
 
+// small_ws: below kLargeMinB rows main_kernel runs, whose workspace is the
+// smaller one.
 static ExactPlan make_exact_plan(int64_t B, int64_t d, int64_t F, int64_t k, int dtype, int ncu,
-                                 const TestHooks& hooks)
+                                 const TestHooks& hooks, bool small_ws = false)
 {
     ExactPlan p;
     p.num_tiles = cdiv(F, kTileLatents);
@@ -267,7 +269,7 @@ static ExactPlan make_exact_plan(int64_t B, int64_t d, int64_t F, int64_t k, int
         // F = 33000 (129 tiles on 128 ranges) 56 / 68, d = 192, F = 24379 36 / 38.  (At up to 256 rows its
         // one row block is no faster at F = 2^16, and its workspace would pass
         // the static scratch of the no-allocation calls.)
-        if (dtype != STK_DTYPE_F32 && B > kLargeRows)
+        if (dtype != STK_DTYPE_F32 && B > kLargeRows && !small_ws)
             p.large = (double)cdiv(p.num_tiles, lnr) * (1.5 * (double)nds + 7.0) + 8.0 < 1.3 * (double)best;
     }
     if (p.large) {
@@ -754,7 +756,8 @@ int stk_exact_forward_noalloc(const void* X, const void* W, const float* b, floa
     int ncu = 0;
     if ((rc = cu_count(&ncu))) return rc;
     const TestHooks hooks = test_hooks();
-    const ExactPlan p = make_exact_plan(B, d, F, k, dtype, ncu, hooks);
+    ExactPlan p = make_exact_plan(B, d, F, k, dtype, ncu, hooks);
+    if (p.total > (size_t)STK_NOALLOC_SCRATCH_BYTES) p = make_exact_plan(B, d, F, k, dtype, ncu, hooks, true);
     if (p.total > (size_t)STK_NOALLOC_SCRATCH_BYTES)
         return set_error(STK_E_WORKSPACE,
                          "this problem needs %zu bytes of workspace, more than the %zu-byte static scratch of "

@@ -11,7 +11,7 @@ import torch
 import oracle
 from hooks import hooks
 from parity import check_against_scores, term_magnitudes, tol_of
-from streamtopk_sae import make_inputs, topk_sae_cuda_exact
+from streamtopk_sae import _lib, make_inputs, topk_sae_cuda_exact
 
 pytestmark = pytest.mark.gpu
 
@@ -95,3 +95,26 @@ def test_split_ignores_values_past_its_rows(cuda_dev):
     for r in rows:
         want = torch.topk(S[r], k).indices
         assert set(I1[r].tolist()) == set(want.tolist())
+
+
+@pytest.mark.parametrize("B,d,F,k", [
+    (300, 256, 65536, 32),    # the large-batch kernel, within the static scratch
+    (400, 64, 262144, 128),   # its workspace would not fit: the other kernel runs
+    (257, 72, 33000, 16),     # 129 tiles
+    (511, 4096, 33000, 64),   # rotated columns of the large-batch kernel
+])
+def test_middle_batches(cuda_dev, B, d, F, k):
+    """Batches of 257 to 511 rows, through the op and without allocation."""
+    print(f"case middle B={B} d={d} F={F} k={k}", flush=True)
+    X, W, b = make_inputs(B, d, F, torch.bfloat16, seed=64, device=cuda_dev)
+    V, I = topk_sae_cuda_exact(X, W, b, k)
+    Vn, In = torch.empty_like(V), torch.empty_like(I)
+    lib = _lib.load()
+    _lib.check(lib.stk_exact_forward_noalloc(X.data_ptr(), W.data_ptr(), b.data_ptr(), Vn.data_ptr(), In.data_ptr(),
+                                             B, d, F, k, _lib.STK_DTYPE_BF16,
+                                             torch.cuda.current_stream().cuda_stream))
+    torch.cuda.synchronize()
+    S = (X.double() @ W.double().T + b.double()).cpu().numpy()
+    A = term_magnitudes(X, W, b)
+    for v, i, name in ((V, I, "middle"), (Vn, In, "middle noalloc")):
+        check_against_scores(v.cpu().numpy(), i.cpu().numpy(), S, k, tol_of("bf16"), name, A=A, d=d)
