@@ -211,7 +211,7 @@ struct ThrArgs {
 // global memory (one segment of `cap` keys per row and W range).
 constexpr int kLargeRows = 256;
 constexpr int kLargeThreads = 256;
-constexpr int64_t kLargeMinB = 512;   // batches from this size use mainl_kernel
+constexpr int64_t kLargeMinB = 512;   // batches from this size use mainl_kernel (from kLargeRows + 1: by estimate)
 // fp32: main_kernel multiplies on the bf16 matrix cores (split3), mainl_kernel
 // on the fp32 ones, at 2.7 times the cycles; past 2048 rows main_kernel's grid
 // has fewer than kXchMinWg workgroups per row block.

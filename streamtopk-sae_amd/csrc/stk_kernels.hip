@@ -1,7 +1,8 @@
 // stk_kernels.hip -- the exact streaming top-k encoder on gfx950.
 //
 //   main_kernel    : streams W once; MFMA scores for 256 latents x up to 128
-//                    rows per tile; scores not below the row threshold go to
+//                    rows per tile (or, d split over the waves, 128 x 64 or
+//                    64 x 32); scores not below the row threshold go to
 //                    a short per-row LDS queue, which spills to the
 //                    workgroup's segment of the row's list when it fills; a
 //                    full segment is rank-compacted to its top-k.  At the end
@@ -148,9 +149,10 @@ __device__ __forceinline__ void flush_rows(int* cnt, int* gcnt, uint64_t* thr, c
 // After the first tile's scores (bias included) are in ac: fills thr[0..BT)
 // with the row thresholds of the exchange.
 //   1. Each workgroup publishes, per row, the score image (ordered_u32) of
-//      the largest score of its first tile (NaN scores left out).
+//      the largest score of each of xper equal parts of its first tile (NaN
+//      scores left out): nw = nwg * xper maxima per row, at most 256.
 //   2. Workgroup x owns rows x, x + nwg, ... of its row block (one wave per
-//      row): once max(k, 3/4 nwg) of the row's maxima have arrived, it takes
+//      row): once max(k, 3/4 nw) of the row's maxima have arrived, it takes
 //      the k-th largest of those: at least k distinct latents of the row
 //      score at least that value, so it is a lower bound of the row's k-th
 //      score, whichever maxima arrived first (the result does not depend on
