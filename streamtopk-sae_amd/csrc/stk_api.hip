@@ -659,6 +659,11 @@ static int validate_approx(int64_t B, int64_t d, int64_t F, int64_t k, int64_t c
                          (long long)c);
     if ((rc = check_shape_common(B, d, F, dtype))) return rc;
     if (k > F) return set_error(STK_E_INVALID, "k out of range");
+    // the kernels address a tile's 256 rows by 32-bit offsets, the upper half
+    // of which stands for "no such chunk"
+    if (d > kMaxRowBytes / (dtype == STK_DTYPE_F32 ? 4 : 2))
+        return set_error(STK_E_INVALID, "d=%lld: rows of more than %lld bytes are not supported", (long long)d,
+                         (long long)kMaxRowBytes);
     return 0;
 }
 

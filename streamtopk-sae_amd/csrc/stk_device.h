@@ -184,7 +184,10 @@ __device__ __forceinline__ uint64_t xch_key(uint32_t T)
 
 // Buffer resource (raw, gfx9 family): loads at byte offsets >= num_records
 // return zeros, which bounds rows past B and latents past F, and a zero-length
-// resource makes whole steps read as zeros.
+// resource makes whole steps read as zeros.  Only the lane's offset is relied
+// on for that: the compiler documents the scalar offset as no part of the
+// check (gfx950 was seen to count both), so what goes there (a column within
+// the row) never passes the end by itself.
 // The streaming kernels build every resource uniform over the wave; its fields
 // go through readfirstlane so that the compiler keeps it in scalar registers
 // whatever its uniformity analysis concludes (a resource it takes for
@@ -499,7 +502,7 @@ struct TileStream {
         return c >= nds ? c - nds : c;
     }
 
-    static constexpr int kOut = 0x40000000;   // an offset beyond every resource (tiles and row blocks: at most 4 MiB)
+    static constexpr int kOut = 0x40000000;   // an offset beyond every resource (at most 256 rows of kMaxRowBytes)
 
     __device__ __forceinline__ void init_x(const unsigned char* X, int64_t B, int64_t b0)
     {
@@ -527,13 +530,13 @@ struct TileStream {
         const int s = col(real ? ls : 0);
         const int so = __builtin_amdgcn_readfirstlane(s * (S * kStepBytes));
         const int to = !real ? kOut : (tail != 0 && s == nds - 1) ? toff : 0;
+        // the rows go into the lane's offset, which the range check covers (see make_rsrc)
+        const int rows = kThr / kRowChunks * (int)w_row_bytes;
 #pragma unroll
-        for (int p = 0; p < kXChunks; ++p)
-            xr[p] = __builtin_amdgcn_raw_buffer_load_b128(xres, xoff + to, so + p * (kThr / kRowChunks) * (int)w_row_bytes, 0);
+        for (int p = 0; p < kXChunks; ++p) xr[p] = __builtin_amdgcn_raw_buffer_load_b128(xres, xoff + to + p * rows, so, 0);
 #pragma unroll
         for (int p = 0; p < kWChunks; ++p)
-            wr[p] = __builtin_amdgcn_raw_buffer_load_b128(wres, woff + to, so + p * (kThr / kRowChunks) * (int)w_row_bytes,
-                                                          NT ? 2 : 0);
+            wr[p] = __builtin_amdgcn_raw_buffer_load_b128(wres, woff + to + p * rows, so, NT ? 2 : 0);
         if (lt < ntiles && ++ls == nds2) {
             ls = 0;
             ++lt;

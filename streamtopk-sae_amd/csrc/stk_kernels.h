@@ -37,6 +37,7 @@ constexpr int kMainWaves = 8;        // wavefronts per main_kernel workgroup (2 
 constexpr int kMainThreads = 64 * kMainWaves;
 constexpr int kTileLatents = 32 * kMainWaves;   // latents per main_kernel tile
 constexpr int kApproxGroup = 128;    // latent group of the approximate variant
+constexpr int64_t kMaxRowBytes = 1 << 22;   // of a row of X or W: 256 of them stay below TileStream::kOut
 constexpr int kRangeUnit = 16;       // main_kernel's workgroups share the latents in units of this many
 constexpr int kGroupTile = 256;      // latents per group_kernel tile (two groups)
 constexpr int kSampleTarget = 4096;  // sampled latents that seed the thresholds

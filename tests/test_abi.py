@@ -127,3 +127,15 @@ def test_merge_workspace_and_errors():
         assert msg in lib.stk_last_error().decode()
     rc = lib.stk_topk_merge(None, None, 2, 4, 8, None, None, None, 0, None)
     assert rc == 1 and "null tensor pointer" in lib.stk_last_error().decode()
+
+
+@pytest.mark.parametrize("dtype,d", [(0, 1 << 20), (2, 1 << 21)])
+def test_approx_rows_within_32bit_offsets(dtype, d):
+    """Rows of 4 MiB are the widest that a tile's 32-bit offsets reach; wider ones are refused before any device work."""
+    lib = _lib.load()
+    step = 4 if dtype == 0 else 8
+    args = [None] * 5
+    assert lib.stk_approx_forward(*args, 4, d + step, 256, 16, 16, dtype, None, None, None, 0, None) == 1
+    assert "rows of more than 4194304 bytes" in lib.stk_last_error().decode()
+    lib.stk_approx_forward(*args, 4, d, 256, 16, 16, dtype, None, None, None, 0, None)
+    assert "null tensor pointer" in lib.stk_last_error().decode()
