@@ -93,9 +93,9 @@ int stk_exact_forward(const void* X, const void* W, const float* b, float* V, in
  * batches of 512 rows and more (config 4) do not.  All calls on one device
  * share its array, so calls that overlap on one device race: serialise them
  * (one stream, or events between streams).  Results are identical to
- * stk_exact_forward's, except that between 257 and 511 rows a problem whose
- * kernel would need more runs the one with the smaller workspace (sums in
- * another order). */
+ * stk_exact_forward's, except that from 257 rows a problem whose kernel would
+ * need more than the array runs the one with the smaller workspace (sums in
+ * another order), and is rejected only if that does not fit either. */
 int stk_exact_forward_noalloc(const void* X, const void* W, const float* b, float* V, int32_t* I,
                               int64_t B, int64_t d, int64_t F, int64_t k, int dtype, void* stream);
 

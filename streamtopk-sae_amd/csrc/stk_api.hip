@@ -196,14 +196,14 @@ struct ExactPlan {
     size_t off_thr, off_list, off_lcnt, off_seg, off_xmax, off_xthr, total;
 };
 
-// small_ws: below kLargeMinB rows main_kernel runs, whose workspace is the
-// smaller one.
+// small_ws: main_kernel runs below kLargeMinB rows and mainl_kernel from there,
+// whatever the type: the smaller workspaces.
 static ExactPlan make_exact_plan(int64_t B, int64_t d, int64_t F, int64_t k, int dtype, int ncu,
                                  const TestHooks& hooks, bool small_ws = false)
 {
     ExactPlan p;
     p.num_tiles = cdiv(F, kTileLatents);
-    p.large = B >= (dtype == STK_DTYPE_F32 ? kLargeMinBF32 : kLargeMinB);
+    p.large = B >= (dtype == STK_DTYPE_F32 && !small_ws ? kLargeMinBF32 : kLargeMinB);
     p.lq = 0;
     p.S = 1;
     p.xper = 1;

@@ -97,24 +97,25 @@ def test_split_ignores_values_past_its_rows(cuda_dev):
         assert set(I1[r].tolist()) == set(want.tolist())
 
 
-@pytest.mark.parametrize("B,d,F,k", [
-    (300, 256, 65536, 32),    # the large-batch kernel, within the static scratch
-    (400, 64, 262144, 128),   # its workspace would not fit: the other kernel runs
-    (257, 72, 33000, 16),     # 129 tiles
-    (511, 4096, 33000, 64),   # rotated columns of the large-batch kernel
+@pytest.mark.parametrize("B,d,F,k,dtype_name", [
+    (300, 256, 65536, 32, "bf16"),    # the large-batch kernel, within the static scratch
+    (400, 64, 262144, 128, "bf16"),   # its workspace would not fit: the other kernel runs
+    (257, 72, 33000, 16, "bf16"),     # 129 tiles
+    (511, 4096, 33000, 64, "bf16"),   # rotated columns of the large-batch kernel
+    (1886, 3656, 18787, 32, "fp32"),  # the streaming kernel's workspace would not fit: the large-batch one runs
 ])
-def test_middle_batches(cuda_dev, B, d, F, k):
-    """Batches of 257 to 511 rows, through the op and without allocation."""
-    print(f"case middle B={B} d={d} F={F} k={k}", flush=True)
-    X, W, b = make_inputs(B, d, F, torch.bfloat16, seed=64, device=cuda_dev)
+def test_middle_batches(cuda_dev, B, d, F, k, dtype_name):
+    """Batches of 257 rows and more, through the op and without allocation."""
+    print(f"case middle {dtype_name} B={B} d={d} F={F} k={k}", flush=True)
+    X, W, b = make_inputs(B, d, F, DT[dtype_name], seed=64, device=cuda_dev)
     V, I = topk_sae_cuda_exact(X, W, b, k)
     Vn, In = torch.empty_like(V), torch.empty_like(I)
     lib = _lib.load()
+    code = {"bf16": _lib.STK_DTYPE_BF16, "fp32": _lib.STK_DTYPE_F32}[dtype_name]
     _lib.check(lib.stk_exact_forward_noalloc(X.data_ptr(), W.data_ptr(), b.data_ptr(), Vn.data_ptr(), In.data_ptr(),
-                                             B, d, F, k, _lib.STK_DTYPE_BF16,
-                                             torch.cuda.current_stream().cuda_stream))
+                                             B, d, F, k, code, torch.cuda.current_stream().cuda_stream))
     torch.cuda.synchronize()
     S = (X.double() @ W.double().T + b.double()).cpu().numpy()
     A = term_magnitudes(X, W, b)
     for v, i, name in ((V, I, "middle"), (Vn, In, "middle noalloc")):
-        check_against_scores(v.cpu().numpy(), i.cpu().numpy(), S, k, tol_of("bf16"), name, A=A, d=d)
+        check_against_scores(v.cpu().numpy(), i.cpu().numpy(), S, k, tol_of(dtype_name), name, A=A, d=d)
