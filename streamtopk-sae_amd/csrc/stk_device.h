@@ -184,10 +184,10 @@ __device__ __forceinline__ uint64_t xch_key(uint32_t T)
 
 // Buffer resource (raw, gfx9 family): loads at byte offsets >= num_records
 // return zeros, which bounds rows past B and latents past F, and a zero-length
-// resource makes whole steps read as zeros.  Only the lane's offset is relied
-// on for that: the compiler documents the scalar offset as no part of the
-// check (gfx950 was seen to count both), so what goes there (a column within
-// the row) never passes the end by itself.
+// resource makes whole steps read as zeros.  The lane's
+// offset is what the compiler documents as checked; gfx950 checks its sum with
+// the scalar one, without wrapping (seen in both kinds of load, for scalar
+// offsets below, at and past num_records).
 // The streaming kernels build every resource uniform over the wave; its fields
 // go through readfirstlane so that the compiler keeps it in scalar registers
 // whatever its uniformity analysis concludes (a resource it takes for
@@ -530,13 +530,18 @@ struct TileStream {
         const int s = col(real ? ls : 0);
         const int so = __builtin_amdgcn_readfirstlane(s * (S * kStepBytes));
         const int to = !real ? kOut : (tail != 0 && s == nds - 1) ? toff : 0;
-        // the rows go into the lane's offset, which the range check covers (see make_rsrc)
+        // the chunks' rows go into the lane's offset, which the range check is
+        // documented to cover; fp32, whose pipeline has no register left for
+        // that (one spilled at 128 rows), into the scalar one, which gfx950
+        // counts as well
         const int rows = kThr / kRowChunks * (int)w_row_bytes;
+        const int vr = kSplit ? 0 : rows, sr = kSplit ? rows : 0;
 #pragma unroll
-        for (int p = 0; p < kXChunks; ++p) xr[p] = __builtin_amdgcn_raw_buffer_load_b128(xres, xoff + to + p * rows, so, 0);
+        for (int p = 0; p < kXChunks; ++p)
+            xr[p] = __builtin_amdgcn_raw_buffer_load_b128(xres, xoff + to + p * vr, so + p * sr, 0);
 #pragma unroll
         for (int p = 0; p < kWChunks; ++p)
-            wr[p] = __builtin_amdgcn_raw_buffer_load_b128(wres, woff + to + p * rows, so, NT ? 2 : 0);
+            wr[p] = __builtin_amdgcn_raw_buffer_load_b128(wres, woff + to + p * vr, so + p * sr, NT ? 2 : 0);
         if (lt < ntiles && ++ls == nds2) {
             ls = 0;
             ++lt;
